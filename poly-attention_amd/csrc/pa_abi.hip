@@ -116,6 +116,7 @@ PassDev to_passdev(const pa_pass* p) {
     P.dim = p->dim;
     P.scale = p->scale;
     P.softclamp = p->softclamp;
+    P.sc = soft_clamp_dev(p->scale, p->softclamp);
     P.causal = p->causal;
     P.flags = p->flags;
     P.q = to_dview(p->q, p->heads);

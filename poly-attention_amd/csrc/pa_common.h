@@ -66,6 +66,32 @@ struct DMask {
     }
 };
 
+// The score soft clamp in units of the raw scores s = q.k (so that scale * log2e times the
+// result is the log2-domain logit): tanh(a s) / a with a = scale / softclamp, by the
+// polynomial s (1 + k1 s^2 + k2 s^4 + k3 s^6) where |s| <= thr.  Filled in by soft_clamp_dev.
+struct SoftClampDev {
+    float k1, k2, k3, thr, a, ia;
+};
+
+// tanh(y) / y on |y| <= 0.35 as 1 + c1 y^2 + c2 y^4 + c3 y^6, fitted for the least maximal
+// relative error (4.1e-8; evaluated in fp32 at most 1.3e-7 off, 4.1e-8 root mean square, as a
+// correctly rounded tanhf is within 6e-8).  A scale or softclamp whose powers leave fp32's range
+// turns the polynomial off (thr < 0: the kernels then take tanhf for every score).
+inline SoftClampDev soft_clamp_dev(float scale, float softclamp) {
+    SoftClampDev c = {0.f, 0.f, 0.f, -1.f, 0.f, 0.f};
+    if (!(softclamp > 0.f)) return c;
+    c.a = scale / softclamp;
+    c.ia = softclamp / scale;
+    const double a2 = (double)c.a * c.a;
+    const double k3 = -4.914850154e-02 * a2 * a2 * a2, thr = 0.35 / fabs((double)c.a);
+    if (!(a2 > 1e-30) || !(fabs(k3) < 1e30) || !(fabs(k3) > 1e-36)) return c;
+    c.k1 = (float)(-3.333266316e-01 * a2);
+    c.k2 = (float)(1.329982537e-01 * a2 * a2);
+    c.k3 = (float)k3;
+    c.thr = (float)thr;
+    return c;
+}
+
 // All the geometry of one pass, as passed to every pass kernel (by value).
 struct PassDev {
     int32_t batch, heads, nq, nk, dim;
@@ -83,6 +109,7 @@ struct PassDev {
     // masked passes on the MFMA kernels: per (b, key head) [first, last + 1) of the keys that
     // can enter a normal row (kept, key bias of class 0), or null
     const int32_t* live;
+    SoftClampDev sc;
 };
 
 struct GradDev {

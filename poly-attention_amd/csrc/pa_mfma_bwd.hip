@@ -180,8 +180,7 @@ __global__ __launch_bounds__(kBwdThreads, D == 64 ? 2 : 1) void k_mfma_bwd_dkv(G
         bias_l2 = bias_class(x) == 0 ? x * kLog2e : -INFINITY;
     }
     const float sl2 = P.scale * kLog2e;
-    const float cinv = SOFTCLAMP ? P.scale / P.softclamp : 0.f;
-    const float crec = SOFTCLAMP ? 1.f / P.softclamp : 0.f;
+    const float ca = SOFTCLAMP ? P.sc.a : 0.f;
 
     f32x16_t dk[D / 32], dv[D / 32];
 #pragma unroll
@@ -223,6 +222,7 @@ __global__ __launch_bounds__(kBwdThreads, D == 64 ? 2 : 1) void k_mfma_bwd_dkv(G
                 }
                 // P: register i holds query qbase + 8*(i/4) + 4*hh + (i%4) of the lane's key
                 float yv[16];
+                if (SOFTCLAMP) soft_clamp16(s, P.sc);
 #pragma unroll
                 for (int g = 0; g < 4; ++g) {
                     const float4 Lv = *reinterpret_cast<const float4*>(sL + qb * 32 + 8 * g + 4 * hh);
@@ -230,14 +230,8 @@ __global__ __launch_bounds__(kBwdThreads, D == 64 ? 2 : 1) void k_mfma_bwd_dkv(G
 #pragma unroll
                     for (int r = 0; r < 4; ++r) {
                         const int i = 4 * g + r;
-                        float x;
-                        if (SOFTCLAMP) {
-                            yv[i] = tanhf(s[i] * cinv);  // softclamp(s*scale) / c
-                            x = yv[i] * (P.softclamp * kLog2e) + bias_l2 - L[r];
-                        } else {
-                            x = fmaf(s[i], sl2, bias_l2 - L[r]);
-                        }
-                        s[i] = fast_exp2(x);
+                        if (SOFTCLAMP) yv[i] = s[i] * ca;  // softclamp(s*scale) / c
+                        s[i] = fast_exp2(fmaf(s[i], sl2, bias_l2 - L[r]));
                     }
                 }
                 if (CAUSAL && qbase < kw0 + 31) {  // queries before the lane's key: P = 0
@@ -278,7 +272,6 @@ __global__ __launch_bounds__(kBwdThreads, D == 64 ? 2 : 1) void k_mfma_bwd_dkv(G
 
     dbias += __shfl_xor(dbias, 32);
     if (!key_ok) return;
-    (void)crec;
     // dK = scale * dK^T^T ; registers: d = x*32 + 8g + 4hh + r
     T* dkrow = G.dk.wrow<T>(b, h0, key);
     T* dvrow = G.dv.wrow<T>(b, h0, key);
@@ -415,8 +408,10 @@ __global__ __launch_bounds__(kBwdThreads, D == 64 ? 2 : 1) void k_mfma_bwd_dkv_d
     }
     bias_l2 = opaque(bias_l2);
     const float sl2 = P.scale * kLog2e;
-    const float cinv = SOFTCLAMP ? P.scale / P.softclamp : 0.f;
-    const float cl2 = SOFTCLAMP ? P.softclamp * kLog2e : 0.f;
+    const float ca = SOFTCLAMP ? P.sc.a : 0.f;
+    // the score of a masked entry: its probability is 0 and, with softclamp, its factor
+    // 1 - (ca s)^2 finite
+    const float masked_s = SOFTCLAMP ? -1e9f / sl2 : -INFINITY;
     const float lmul = SOFTCLAMP ? kLog2e : -1.f / P.scale;  // lse -> seed / log2 value
     const bool need_dbias = G.dbias.ok();
 
@@ -582,7 +577,7 @@ __global__ __launch_bounds__(kBwdThreads, D == 64 ? 2 : 1) void k_mfma_bwd_dkv_d
 #pragma unroll
                 for (int i = 0; i < 16; ++i) {
                     const int o = 8 * (i / 4) + (i % 4);
-                    if (o < lo || o >= hi) s[i] = -INFINITY;
+                    if (o < lo || o >= hi) s[i] = masked_s;
                 }
             }
         };
@@ -598,8 +593,8 @@ __global__ __launch_bounds__(kBwdThreads, D == 64 ? 2 : 1) void k_mfma_bwd_dkv_d
 #pragma unroll
                     for (int r = 0; r < 4; ++r) {
                         const int i = 4 * g + r;
-                        yv[i] = s[i] == -INFINITY ? 1.f : tanhf(s[i] * cinv);
-                        s[i] = s[i] == -INFINITY ? 0.f : fast_exp2(yv[i] * cl2 + bias_l2 - L[r]);
+                        yv[i] = s[i] * ca;
+                        s[i] = fast_exp2(fmaf(s[i], sl2, bias_l2 - L[r]));
                     }
                 }
             } else {
@@ -638,9 +633,14 @@ __global__ __launch_bounds__(kBwdThreads, D == 64 ? 2 : 1) void k_mfma_bwd_dkv_d
         f32x16_t s0, dp0, s1, dp1;
         frag pf0[2], df0[2], pf1[2], df1[2];
         scores(0, s0, dp0);
-        mask(0, s0);
+        if (!SOFTCLAMP) mask(0, s0);
         scores(1, s1, dp1);
+        if (SOFTCLAMP) {
+            soft_clamp16(s0, P.sc);
+            mask(0, s0);
+        }
         grads(0, s0, dp0, pf0, df0);
+        if (SOFTCLAMP) soft_clamp16(s1, P.sc);
         mask(1, s1);
         accumulate(0, pf0, df0);
         grads(1, s1, dp1, pf1, df1);
@@ -830,7 +830,7 @@ __global__ __launch_bounds__(kBwdThreads, D == 64 ? 2 : 1) void k_mfma_bwd_dq(Gr
     const float lse_l2 = q_ok ? G.ws_lse[row] * kLog2e : INFINITY;
     const float dpi = q_ok ? G.ws_D[row] : 0.f;
     const float sl2 = P.scale * kLog2e;
-    const float cinv = SOFTCLAMP ? P.scale / P.softclamp : 0.f;
+    const float ca = SOFTCLAMP ? P.sc.a : 0.f;
 
     f32x16_t dq[D / 32];
 #pragma unroll
@@ -862,6 +862,7 @@ __global__ __launch_bounds__(kBwdThreads, D == 64 ? 2 : 1) void k_mfma_bwd_dq(Gr
                 }
                 // P^T: register i holds key j0 + kb*32 + 8*(i/4) + 4*hh + (i%4) of the lane's query
                 float yv[16];
+                if (SOFTCLAMP) soft_clamp16(s, P.sc);
 #pragma unroll
                 for (int g = 0; g < 4; ++g) {
                     const float4 bb = *reinterpret_cast<const float4*>(sB + kb * 32 + 8 * g + 4 * hh);
@@ -869,14 +870,8 @@ __global__ __launch_bounds__(kBwdThreads, D == 64 ? 2 : 1) void k_mfma_bwd_dq(Gr
 #pragma unroll
                     for (int r = 0; r < 4; ++r) {
                         const int i = 4 * g + r;
-                        float x;
-                        if (SOFTCLAMP) {
-                            yv[i] = tanhf(s[i] * cinv);
-                            x = yv[i] * (P.softclamp * kLog2e) + bv[r] - lse_l2;
-                        } else {
-                            x = fmaf(s[i], sl2, bv[r] - lse_l2);
-                        }
-                        s[i] = fast_exp2(x);
+                        if (SOFTCLAMP) yv[i] = s[i] * ca;
+                        s[i] = fast_exp2(fmaf(s[i], sl2, bv[r] - lse_l2));
                     }
                 }
                 if (diag) {  // keys after the lane's query: P = 0
@@ -930,8 +925,9 @@ __global__ __launch_bounds__(kBwdThreads, D == 64 ? 2 : 1) void k_mfma_bwd_dq(Gr
 // converts the tile's key bias into accumulator seeds (bias / scale; log2 domain with
 // softclamp), so that P^T = exp2(scale*log2e*S^T - lse*log2e).  Three workgroups per CU at
 // head dim 64 (the register budget fits without spills).
+// (two workgroups per CU with softclamp: at three, 27 to 62 of its registers spill)
 template <typename T, int D, bool CAUSAL, bool SOFTCLAMP, bool HAS_BIAS>
-__global__ __launch_bounds__(kBwdThreads, D == 64 ? 3 : 1) void k_mfma_bwd_dq_dma(GradDev G) {
+__global__ __launch_bounds__(kBwdThreads, D == 64 ? (SOFTCLAMP ? 2 : 3) : 1) void k_mfma_bwd_dq_dma(GradDev G) {
     using M = Mma<T>;
     typedef typename M::frag frag;
     constexpr int BN = kDqBN, CPR = D / 8, ELEMS = BN * D;
@@ -1023,8 +1019,10 @@ __global__ __launch_bounds__(kBwdThreads, D == 64 ? 3 : 1) void k_mfma_bwd_dq_dm
     lse_l2 = opaque(lse_l2);
     dpi = opaque(dpi);
     const float sl2 = P.scale * kLog2e;
-    const float cinv = SOFTCLAMP ? P.scale / P.softclamp : 0.f;
-    const float cl2 = SOFTCLAMP ? P.softclamp * kLog2e : 0.f;
+    const float ca = SOFTCLAMP ? P.sc.a : 0.f;
+    // the score of a masked entry: its probability is 0 and, with softclamp, its factor
+    // 1 - (ca s)^2 finite
+    const float masked_s = SOFTCLAMP ? -1e9f / sl2 : -INFINITY;
 
     f32x16_t dq[D / 32];
 #pragma unroll
@@ -1154,7 +1152,7 @@ __global__ __launch_bounds__(kBwdThreads, D == 64 ? 3 : 1) void k_mfma_bwd_dq_dm
                 lim -= 4 * hh;
 #pragma unroll
                 for (int i = 0; i < 16; ++i)
-                    if (8 * (i / 4) + (i % 4) > lim) s[i] = -INFINITY;
+                    if (8 * (i / 4) + (i % 4) > lim) s[i] = masked_s;
             }
         };
         // dS^T = P^T (dP^T - D), packed as B operands
@@ -1174,8 +1172,8 @@ __global__ __launch_bounds__(kBwdThreads, D == 64 ? 3 : 1) void k_mfma_bwd_dq_dm
 #pragma unroll
                     for (int r = 0; r < 4; ++r) {
                         const int i = 4 * g + r;
-                        yv[i] = s[i] == -INFINITY ? 1.f : tanhf(s[i] * cinv);
-                        s[i] = s[i] == -INFINITY ? 0.f : fast_exp2(yv[i] * cl2 + bv[r] - lse_l2);
+                        yv[i] = s[i] * ca;
+                        s[i] = fast_exp2(fmaf(s[i], sl2, bv[r] - lse_l2));
                     }
                 }
             } else {
@@ -1298,9 +1296,14 @@ __global__ __launch_bounds__(kBwdThreads, D == 64 ? 3 : 1) void k_mfma_bwd_dq_dm
         }
 #endif
         scores(0, s0, dp0);
-        mask(0, s0);
+        if (!SOFTCLAMP) mask(0, s0);
         scores(1, s1, dp1);
+        if (SOFTCLAMP) {
+            soft_clamp16(s0, P.sc);
+            mask(0, s0);
+        }
         grads(0, s0, dp0, df0);
+        if (SOFTCLAMP) soft_clamp16(s1, P.sc);
         mask(1, s1);
         accumulate(0, df0);
         grads(1, s1, dp1, df1);

@@ -242,13 +242,20 @@ struct FwdWave {
     using M = Mma<T>;
     typedef typename M::frag frag;
     static constexpr int BN = TL::BN;
-    static constexpr bool PLAIN = !BIAS_IN_LOGITS && !SOFTCLAMP;  // max taken on raw scores
+    static constexpr bool PLAIN = !BIAS_IN_LOGITS;  // max taken on raw (soft-clamped) scores
 
     frag qf[D / 16];
     f32x16_t o[D / 32];
     float m, l;
     int kcol, hh, q0, qi, nk;
-    float sl2, cinv, cl2;
+    float sl2;
+
+    // softclamp of the raw scores, before any masking (clamp-free kernels: nothing)
+    __device__ __forceinline__ void clamp(f32x16_t (&s)[KB], const PassDev& P) const {
+        if constexpr (SOFTCLAMP)
+#pragma unroll
+            for (int kb = 0; kb < KB; ++kb) soft_clamp16(s[kb], P.sc);
+    }
 
     // S^T block kb of a key tile: s[kb] = K[kb*32 + row, :] . Q^T
     __device__ __forceinline__ void scores(const T* K, f32x16_t (&s)[KB]) const {
@@ -292,7 +299,7 @@ struct FwdWave {
         }
     }
 
-    // scores -> log2-domain logits in place (bias / softclamp paths); returns the max over the
+    // (soft-clamped) scores -> log2-domain logits in place (bias path); returns the max over the
     // query's logits of this tile (PLAIN: of the raw scores, times scale*log2e)
     __device__ __forceinline__ float logits(f32x16_t (&s)[KB], const float* sB) const {
         // four independent max chains (short dependency chains), combined at the end
@@ -313,8 +320,7 @@ struct FwdWave {
                 for (int r = 0; r < 4; ++r) {
                     float x = s[kb][4 * g + r];
                     if (!PLAIN) {
-                        if (SOFTCLAMP) x = (x == -INFINITY) ? -INFINITY : cl2 * tanhf(x * cinv) + bv[r];
-                        else x = fmaf(x, sl2, bv[r]);
+                        x = fmaf(x, sl2, bv[r]);
                         s[kb][4 * g + r] = x;
                     }
                     mq[r] = fmaxf(mq[r], x);
@@ -437,8 +443,6 @@ __global__ __launch_bounds__(kFwdThreads, D == 64 ? 2 : 1) void k_mfma_fwd(PassD
     wv.qi = wv.q0 + wv.kcol;
     wv.nk = P.nk;
     wv.sl2 = P.scale * kLog2e;
-    wv.cinv = SOFTCLAMP ? P.scale / P.softclamp : 0.f;
-    wv.cl2 = SOFTCLAMP ? P.softclamp * kLog2e : 0.f;
     wv.m = -INFINITY;
     wv.l = 0.f;
     // Q^T operand fragments: lane (q, hh) holds Q[q][c*16 + 8*hh .. +7]
@@ -473,6 +477,7 @@ __global__ __launch_bounds__(kFwdThreads, D == 64 ? 2 : 1) void k_mfma_fwd(PassD
 
     f32x16_t sa[KB], sb[KB];
     wv.scores(sK[0], sa);
+    wv.clamp(sa, P);
     wv.mask_edges(sa, 0);
 
     // one pipeline step: softmax + PV of tile t (scores in `cur`), scores of tile t+1 into `nxt`
@@ -493,7 +498,10 @@ __global__ __launch_bounds__(kFwdThreads, D == 64 ? 2 : 1) void k_mfma_fwd(PassD
             wv.load_v(sVt[t & 1], vf);
             wv.l += wv.probs(cur, wv.m == -INFINITY ? 0.f : wv.m, pk);
             wv.pv(vf, pk);
-            if (act_next) wv.mask_edges(nxt, j0 + BN);
+            if (act_next) {
+                wv.clamp(nxt, P);
+                wv.mask_edges(nxt, j0 + BN);
+            }
         }
         fwd_store<T, D, KB, HAS_BIAS>(st, sK[t & 1], more_k, sVt[(t + 1) & 1], sB[(t + 1) & 1], more_v);
         __syncthreads();
@@ -572,10 +580,11 @@ template <typename T, int D, int KB, int QB, bool CAUSAL, bool SOFTCLAMP, bool H
 __global__ __launch_bounds__(kFwdThreads, D == 64 ? 2 : 1) void k_mfma_fwd_dma(PassDev P) {
     using TL = DmaTile<D, KB>;
     constexpr int BN = TL::BN, NL = TL::NL, BM = kFwdBM * QB;
-    // without softclamp the key bias enters the scores as the MFMA accumulator's initial value
-    // (bias / scale, so that scale*log2e*(s + bias/scale) is the log2-domain logit)
+    // the key bias enters the scores as bias / scale (so that scale*log2e*(s + bias/scale) is the
+    // log2-domain logit): as the MFMA accumulator's initial value, with softclamp as the
+    // addend of its last step
     constexpr bool FOLD = HAS_BIAS && !SOFTCLAMP;
-    using W = FwdWave<T, D, KB, CAUSAL, SOFTCLAMP, HAS_BIAS, HAS_BIAS && SOFTCLAMP>;
+    using W = FwdWave<T, D, KB, CAUSAL, SOFTCLAMP, HAS_BIAS, false>;
     using M = Mma<T>;
     typedef typename W::frag frag;
     constexpr int NSTG = kFwdStages;
@@ -603,8 +612,6 @@ __global__ __launch_bounds__(kFwdThreads, D == 64 ? 2 : 1) void k_mfma_fwd_dma(P
         v.qi = v.q0 + kcol;
         v.nk = P.nk;
         v.sl2 = P.scale * kLog2e;
-        v.cinv = SOFTCLAMP ? P.scale / P.softclamp : 0.f;
-        v.cl2 = SOFTCLAMP ? P.softclamp * kLog2e : 0.f;
         v.m = -INFINITY;
         v.l = 0.f;
         const int qi = v.qi;
@@ -632,7 +639,7 @@ __global__ __launch_bounds__(kFwdThreads, D == 64 ? 2 : 1) void k_mfma_fwd_dma(P
     const srd_t rk = make_srd(P.k.row<T>(b, h, 0), (uint32_t)(((int64_t)(P.nk - 1) * ksn + D) * 2));
     const srd_t rv = make_srd(P.v.row<T>(b, h, 0), (uint32_t)(((int64_t)(P.nk - 1) * vsn + D) * 2));
     const int bes = P.bias.dtype == PA_F32 ? 4 : 2;  // bias element size
-    const float bmul = FOLD ? 1.f / P.scale : kLog2e;
+    const float bmul = 1.f / P.scale;
     srd_t rb = {0, 0, 0, 0};
     if (HAS_BIAS) rb = make_srd(P.bias.p + P.bias.idx(b, h, 0) * bes, (uint32_t)(P.nk * bes));
     // per-thread byte offsets (tile-relative) of the chunks this thread loads: chunk
@@ -710,14 +717,23 @@ __global__ __launch_bounds__(kFwdThreads, D == 64 ? 2 : 1) void k_mfma_fwd_dma(P
         if (u + 2 < ntl) issue((tb + u + 2) * BN, (st + 2) & 3);
         if (u + 3 < ntl) issue((tb + u + 3) * BN, (st + 3) & 3);
     };
+    // softclamp (and the key bias) on a block's raw scores, before any masking
+    auto clamp = [&](f32x16_t (&s)[KB]) __attribute__((always_inline)) {
+        if constexpr (SOFTCLAMP)
+#pragma unroll
+            for (int kb = 0; kb < KB; ++kb)
+                soft_clamp16(s[kb], P.sc, [&](int g) __attribute__((always_inline)) {
+                    if (!HAS_BIAS) return make_float4(0.f, 0.f, 0.f, 0.f);
+                    return *reinterpret_cast<const float4*>(&sBw[w][kb * 32 + 8 * g + 4 * hh]);
+                });
+    };
     for (int u = 0; u < nact; ++u) {
         const int j0 = (tb + u) * BN;
         enter(u);
         const T* K = sK + st * TL::ELEMS;
         const T* V = sV + st * TL::ELEMS;
         if (HAS_BIAS) {
-            // this wave's converted copy of the tile's bias: class filtered; log2 domain
-            // (softclamp) or divided by the scale (folded into the scores)
+            // this wave's converted copy of the tile's bias: class filtered, divided by the scale
             float x;
             if (bes == 4) x = sBraw[st][lane];
             else x = (float)reinterpret_cast<const T*>(&sBraw[st][0])[lane];
@@ -789,6 +805,7 @@ __global__ __launch_bounds__(kFwdThreads, D == 64 ? 2 : 1) void k_mfma_fwd_dma(P
             for (int c = 0; c < D / 16; ++c)
 #pragma unroll
                 for (int kb = 0; kb < KB; ++kb) s[0][kb] = M::run(kf[kb][c], wv[0].qf[c], s[0][kb]);
+            clamp(s[0]);
             wv[0].mask_edges_nk(s[0], j0);
             // the first tile: O and l are still 0, so the running max is just the tile's (no
             // attempt against m = -inf that the sum check would send back)
@@ -823,6 +840,7 @@ __global__ __launch_bounds__(kFwdThreads, D == 64 ? 2 : 1) void k_mfma_fwd_dma(P
                         vf[kb][t2][x] = __builtin_bit_cast(frag, v4);
                     }
             recheck(0, lt0, pk0);
+            clamp(s[1]);
             wv[1].mask_edges_nk(s[1], j0);
             if (u == 0) wv[1].m = wv[1].logits(s[1], sBw[w]);
             __builtin_amdgcn_sched_barrier(0);
@@ -874,6 +892,7 @@ __global__ __launch_bounds__(kFwdThreads, D == 64 ? 2 : 1) void k_mfma_fwd_dma(P
         constexpr bool SUMCHK = PA_FWD_SUMCHECK && W::PLAIN;
 #pragma unroll
         for (int u = 0; u < QB; ++u) {
+            clamp(s[u]);
             wv[u].mask_edges_nk(s[u], j0);
             if (!SUMCHK) wv[u].settle(wv[u].logits(s[u], sBw[w]));
         }
@@ -1040,7 +1059,7 @@ __device__ __forceinline__ void norm_row_chunk(u32x4_t& k, const float (&w)[8], 
 template <typename T, class W>
 __device__ __forceinline__ void short_block(W& wv, const PassDev& P, int q0, int lane,
                                             const u32x4_t (&q)[4], const T* Ks, const T* Vt,
-                                            const float* Bk, bool softclamp) {
+                                            const float* Bk) {
     constexpr int D = 64, KB = 2;
     typedef typename W::frag frag;
     wv.hh = lane >> 5;
@@ -1049,8 +1068,6 @@ __device__ __forceinline__ void short_block(W& wv, const PassDev& P, int q0, int
     wv.qi = q0 + wv.kcol;
     wv.nk = P.nk;
     wv.sl2 = P.scale * kLog2e;
-    wv.cinv = softclamp ? P.scale / P.softclamp : 0.f;
-    wv.cl2 = softclamp ? P.softclamp * kLog2e : 0.f;
     wv.m = -INFINITY;
     wv.l = 0.f;
 #pragma unroll
@@ -1059,6 +1076,7 @@ __device__ __forceinline__ void short_block(W& wv, const PassDev& P, int q0, int
     for (int x = 0; x < D / 32; ++x) wv.o[x] = zero16();
     f32x16_t s[KB];
     wv.scores(Ks, s);
+    wv.clamp(s, P);
     wv.mask_edges(s, 0);
     wv.settle(wv.logits(s, Bk));
     u32x4_t pk[KB][2];
@@ -1195,7 +1213,7 @@ __global__ __launch_bounds__(kFwdThreads, 2) void k_mfma_fwd_short(PassDev P) {
     for (int u = 0; u < QPW; ++u) {  // this wave's 32-query blocks
         if (32 * (qb0 + u) >= P.nq) break;  // wave-uniform
         W wv;
-        short_block<T>(wv, P, 32 * (qb0 + u), lane, qraw[u], Ks, Vt, Bk, SOFTCLAMP);
+        short_block<T>(wv, P, 32 * (qb0 + u), lane, qraw[u], Ks, Vt, Bk);
         u32x2_t ow[D / 8];
         short_finish<T>(wv, P, b, h, true, ow);
     }
@@ -1301,7 +1319,7 @@ __global__ __launch_bounds__(kFwdThreads, 2) void k_mfma_order2_short(PassDev P1
     const bool run1 = 32 * p < n2;  // wave-uniform
     if (run1) {
         W1 wv;
-        short_block<T>(wv, P1, 32 * p, lane, q2r, sK1[slot], sVt1[slot], nullptr, SOFTCLAMP);
+        short_block<T>(wv, P1, 32 * p, lane, q2r, sK1[slot], sVt1[slot], nullptr);
         lse = short_finish<T>(wv, P1, b, h, live && !(P1.flags & PA_FLAG_DISCARD_OUT), ow);
     }
     {
@@ -1325,7 +1343,7 @@ __global__ __launch_bounds__(kFwdThreads, 2) void k_mfma_order2_short(PassDev P1
     // pass 2 for q1 block p
     if (32 * p < P2.nq) {
         W2 wv;
-        short_block<T>(wv, P2, 32 * p, lane, q1r, sK2[slot], sVt2[slot], sB2[slot], SOFTCLAMP);
+        short_block<T>(wv, P2, 32 * p, lane, q1r, sK2[slot], sVt2[slot], sB2[slot]);
         u32x2_t ow2[D / 8];
         short_finish<T>(wv, P2, b, h, live, ow2);
     }
