@@ -1,0 +1,78 @@
+"""The fp32 passes on the bf16 matrix cores (three-way operand split): every workgroup shape of the
+dispatch (row blocks per workgroup x waves per row block) at the edges of its tiles, against the
+oracle at 1e-4, the split's accuracy against 64 bits, and infinite inputs."""
+
+import pytest
+import torch
+
+import oracle.poly_oracle as O
+from test_gpu_1_pass import check, dev, randn, run_pass
+
+pytestmark = pytest.mark.gpu
+param = pytest.mark.parametrize
+
+
+@param("n", (1, 31, 33, 64, 65, 129))
+@param("d", (64, 128))
+def test_small_grids(n, d):
+    """Two row blocks and (d = 64) four or (d = 128) two waves each; up to one row past a tile, a
+    row block and a stage; causal, GQA, key bias and value multiplier."""
+    q = randn((1, 4, n, d), torch.float32, 1)
+    k, v, vmul = (randn((1, 2, n, d), torch.float32, s) for s in (2, 3, 4))
+    bias = randn((1, 2, n), torch.float32, 5)
+    check(run_pass(q, k, v, vmul=vmul, bias=bias, causal=True), torch.float32, f"n={n} d={d}")
+
+
+@param("units,n,d,causal", ((128, 130, 64, False), (256, 130, 64, True), (256, 257, 64, True),
+                            (128, 130, 128, False), (256, 129, 128, True)))
+def test_large_grids(units, n, d, causal):
+    """Four and eight row blocks per workgroup, the last one partly empty."""
+    q, k, v = (randn((units // 16, 16, n, d), torch.float32, s) for s in (6, 7, 8))
+    check(run_pass(q, k, v, causal=causal), torch.float32, f"units={units} n={n} d={d}")
+
+
+def _pass64(q, k, v, do):
+    ts = [t.double().requires_grad_() for t in (q, k, v)]
+    out, _ = O.attn_pass(*ts, causal=True)
+    return [out.detach(), *torch.autograd.grad(out, ts, do.double())]
+
+
+@param("scale", (1.0, 1e-6, 1e4))
+def test_accuracy_against_64_bits(scale):
+    """Values of every magnitude split alike: relative error (2-norm) at most 2e-6, four times the
+    largest that fp32 products showed at this size (the sums are 300 terms of fp32)."""
+    from poly_attention import _ops
+
+    q, k, v, do = (randn((1, 4, 300, 64), torch.float32, s) for s in (9, 10, 11, 12))
+    v, do = v * scale, do / scale
+    ts = [t.to(dev()).requires_grad_() for t in (q, k, v)]
+    out, _ = _ops.attn_pass(*ts, causal=True)
+    got = [out.detach(), *torch.autograd.grad(out, ts, do.to(dev()))]
+    for a, b in zip(got, _pass64(q, k, v, do)):
+        assert ((a.double().cpu() - b).norm() / b.norm()).item() < 2e-6
+
+
+@param("d", (64, 128))
+def test_infinite_and_huge_values(d):
+    """An infinite value element reaches every row that attends its key as +-inf in that feature and
+    nowhere else, as with fp32 products; a finite value above bf16's largest number stays finite."""
+    from poly_attention import _ops
+
+    n = 70
+    q, k, v = (randn((1, 2, n, d), torch.float32, s) for s in (13, 14, 15))
+    v[0, 0, 40, 5] = float("inf")
+    v[0, 1, 40, 9] = 3.4e38
+    out, lse = _ops.attn_pass(*(t.to(dev()) for t in (q, k, v)), causal=False)
+    ref, ref_lse = O.attn_pass(q.double(), k.double(), v.double(), causal=False)
+    out = out.cpu().double()
+    inf = torch.isinf(ref)
+    assert inf.any() and torch.equal(torch.isinf(out), inf) and (out[inf] > 0).all()
+    assert torch.isfinite(out[~inf]).all()
+    assert ((out[~inf] - ref[~inf]).abs() <= 1e-4 + 1e-5 * ref[~inf].abs()).all()
+    assert torch.allclose(lse.cpu().double(), ref_lse, atol=1e-4)
+    # causal: the rows before the key, in the features without an infinity (in feature 5 the eager
+    # reference multiplies it by the masked probability 0)
+    out, _ = _ops.attn_pass(*(t.to(dev()) for t in (q, k, v)), causal=True)
+    ref, _ = O.attn_pass(q.double(), k.double(), v.double(), causal=True)
+    rows, feats = slice(0, 32), [f for f in range(d) if f != 5]
+    assert ((out[0, 0, rows, feats].cpu().double() - ref[0, 0, rows, feats]).abs() <= 1e-4).all()
