@@ -71,6 +71,9 @@ extern "C" {
 
 /* pa_pass.flags */
 #define PA_FLAG_MAY_DEGENERATE 1   /* masks or -FLT_MAX biases may leave rows fully masked */
+#define PA_FLAG_BIAS_PADDED    8   /* each fp32 bias row may be read (not used) up to the next multiple
+                                      of 4 elements: lets lengths that are not one take the
+                                      direct-to-LDS kernels */
 #define PA_FLAG_DISCARD_OUT    4   /* pa_poly_order2_fwd, first pass: the caller does not read its
                                       out and lse, which the one-launch path then leaves unwritten
                                       (the buffers are still required) */

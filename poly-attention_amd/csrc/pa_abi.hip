@@ -173,6 +173,10 @@ bool pass_masked(const pa_pass& f) {
 // key-term row stride: whole 16-byte chunks
 int key_term_stride(const pa_pass& f) { return (f.nk + 3) & ~3; }
 
+// row stride of the backward's per-row values (GradDev::rsn): whole 16-byte chunks, so that the
+// direct-to-LDS dK/dV kernel takes every length
+int bwd_row_stride(const pa_pass& f) { return (f.nq + 3) & ~3; }
+
 size_t elem_bytes(int dtype) { return dtype == PA_F32 ? 4 : 2; }
 
 // forward workspace: the per-key term of a key-masked 16-bit pass on the MFMA kernels, whose
@@ -191,7 +195,7 @@ size_t fwd_ws_bytes(const pa_pass& f) {
 // per-key-head bias-class counts and the per-key-head range of keys that can enter a normal row
 size_t bwd_ws_bytes(const pa_pass& f) {
     const size_t rows = (size_t)f.batch * f.heads * f.nq;
-    size_t n = 3 * align256(rows * sizeof(float));
+    size_t n = 3 * align256((size_t)f.batch * f.heads * bwd_row_stride(f) * sizeof(float));
     if (f.epi) n += align256(rows * f.dim * elem_bytes(f.q.dtype));
     if (pass_masked(f)) {
         const size_t kheads = (size_t)f.batch * f.k.heads;
@@ -375,6 +379,7 @@ int pa_attn_pass_fwd(const pa_pass* p, void* stream) {
             PassDev Pm = P;
             Pm.bias = DView{reinterpret_cast<char*>(kterm), (int64_t)hk * nkp, nkp, 1,
                             p->heads / hk, PA_F32};
+            Pm.flags |= PA_FLAG_BIAS_PADDED;
             Pm.km.p = nullptr;
             Pm.live = live;
             launch_mfma_fwd(Pm, T, s);
@@ -467,11 +472,13 @@ int pa_attn_pass_bwd(const pa_pass_grad* g, void* stream) {
     G.accumulate = g->accumulate;
     G.hk = hk;
     const size_t rows = (size_t)p->batch * H * p->nq;
+    G.rsn = bwd_row_stride(*p);
+    const size_t rbytes = align256((size_t)p->batch * H * G.rsn * sizeof(float));
     char* ws = static_cast<char*>(g->workspace);
     G.ws_D = reinterpret_cast<float*>(ws);
-    G.ws_lse = reinterpret_cast<float*>(ws + align256(rows * sizeof(float)));
-    G.ws_invc = reinterpret_cast<float*>(ws + 2 * align256(rows * sizeof(float)));
-    ws += 3 * align256(rows * sizeof(float));
+    G.ws_lse = reinterpret_cast<float*>(ws + rbytes);
+    G.ws_invc = reinterpret_cast<float*>(ws + 2 * rbytes);
+    ws += 3 * rbytes;
     const pa_view none = {};
     G.droot = to_dview(p->epi ? g->droot : none, H);
     G.dgate = to_dview(p->epi ? g->dgate : none, H);
@@ -514,6 +521,7 @@ int pa_attn_pass_bwd(const pa_pass_grad* g, void* stream) {
         G.ws_kcnt = kcnt;
         launch_key_terms(G, kterm, nkp, kcnt, live, s);
         GradDev Gm = G;
+        Gm.f.flags &= ~PA_FLAG_MAY_DEGENERATE;
         if (kterm) {
             DView& kb = Gm.f.bias;
             kb.p = reinterpret_cast<char*>(kterm);
@@ -522,10 +530,10 @@ int pa_attn_pass_bwd(const pa_pass_grad* g, void* stream) {
             kb.sn = 1;
             kb.hdiv = H / hk;
             kb.dtype = PA_F32;
+            Gm.f.flags |= PA_FLAG_BIAS_PADDED;
         }
         Gm.f.km.p = nullptr;
         Gm.f.qm.p = nullptr;
-        Gm.f.flags &= ~PA_FLAG_MAY_DEGENERATE;
         Gm.f.live = live;
         // the direct-to-LDS dQ kernel does the preprocess of the normal rows where it applies
         // (fully-masked rows get lse +inf there: no normal entry; k_fix_rows does the rest of

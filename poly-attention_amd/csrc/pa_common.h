@@ -118,9 +118,10 @@ struct GradDev {
     DView droot, dgate;    // epilogue input gradients (with f.ey)
     int32_t accumulate;
     int32_t hk;            // key-side head count (k, v, vmul, bias share it)
-    float* ws_D;           // [B, heads, nq]  rowsum(dO * O) - dlse
-    float* ws_lse;         // [B, heads, nq]  lse for normal rows, +inf for degenerate rows
-    float* ws_invc;        // [B, heads, nq]  1 / (#class-1 keys) for degenerate rows, else 0
+    int32_t rsn;           // row stride of the next three: nq in whole 16-byte chunks
+    float* ws_D;           // [B, heads, rsn]  rowsum(dO * O) - dlse
+    float* ws_lse;         // [B, heads, rsn]  lse for normal rows, +inf for degenerate rows
+    float* ws_invc;        // [B, heads, rsn]  1 / (#class-1 keys) for degenerate rows, else 0
     int32_t fused_pre;     // the dQ kernel computes ws_D / ws_lse for its rows (no preprocess)
     int32_t seeds;         // with fused_pre: ws_lse / ws_D hold the dK/dV kernel's accumulator
                            // seeds, -lse/scale (lse*log2e with softclamp) and -D

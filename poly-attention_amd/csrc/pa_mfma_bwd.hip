@@ -72,7 +72,7 @@ __device__ __forceinline__ QuerySide<T> query_side(const GradDev& G, int b, int 
     s.dout = G.dout.row<T>(b, h, 0);
     s.qsn = P.q.sn;
     s.osn = G.dout.sn;
-    const int64_t row0 = ((int64_t)b * P.heads + h) * P.nq;
+    const int64_t row0 = ((int64_t)b * P.heads + h) * G.rsn;
     s.lse = G.ws_lse + row0;
     s.dsum = G.ws_D + row0;
     s.nq = P.nq;
@@ -460,9 +460,9 @@ __global__ __launch_bounds__(kBwdThreads, D == 64 ? 2 : 1) void k_mfma_bwd_dkv_d
     auto set_head = [&](int h) __attribute__((always_inline)) {
         rq = make_srd(P.q.row<T>(b, h, 0), qbytes);
         ro = make_srd(G.dout.row<T>(b, h, 0), obytes);
-        const int64_t row0 = ((int64_t)b * P.heads + h) * P.nq;
-        rl = make_srd(G.ws_lse + row0, (uint32_t)(P.nq * 4));
-        rd = make_srd(G.ws_D + row0, (uint32_t)(P.nq * 4));
+        const int64_t row0 = ((int64_t)b * P.heads + h) * G.rsn;
+        rl = make_srd(G.ws_lse + row0, (uint32_t)(G.rsn * 4));
+        rd = make_srd(G.ws_D + row0, (uint32_t)(G.rsn * 4));
     };
     set_head(h0);
     auto issue = [&](int stage) __attribute__((always_inline)) {
@@ -826,7 +826,7 @@ __global__ __launch_bounds__(kBwdThreads, D == 64 ? 2 : 1) void k_mfma_bwd_dq(Gr
         qf[c] = __builtin_bit_cast(frag, qr);
         of[c] = __builtin_bit_cast(frag, orr);
     }
-    const int64_t row = ((int64_t)b * P.heads + h) * P.nq + (q_ok ? qi : 0);
+    const int64_t row = ((int64_t)b * P.heads + h) * G.rsn + (q_ok ? qi : 0);
     const float lse_l2 = q_ok ? G.ws_lse[row] * kLog2e : INFINITY;
     const float dpi = q_ok ? G.ws_D[row] : 0.f;
     const float sl2 = P.scale * kLog2e;
@@ -973,7 +973,7 @@ __global__ __launch_bounds__(kBwdThreads, D == 64 ? (SOFTCLAMP ? 2 : 3) : 1) voi
         l = *P.lse.row<float>(b, h, qc);
         if (G.dlse.ok()) dl = *G.dlse.row<float>(b, h, qc);
     }
-    const int64_t row = ((int64_t)b * P.heads + h) * P.nq + qc;
+    const int64_t row = ((int64_t)b * P.heads + h) * G.rsn + qc;
     float lse_l2, dpi;
     if (G.fused_pre) {
         // the preprocess of this wave's rows: D = rowsum(dO * O) - dlse, lse (+inf for a
@@ -997,13 +997,16 @@ __global__ __launch_bounds__(kBwdThreads, D == 64 ? (SOFTCLAMP ? 2 : 3) : 1) voi
         const float lseb = normal ? l : INFINITY;
         dpi = normal ? dsum - dl : 0.f;
         lse_l2 = q_ok ? lseb * kLog2e : INFINITY;
-        if (q_ok && hh == 0) {
+        // (rows up to rsn: the dK/dV kernel loads whole chunks, whose rows past the end must hold
+        // finite values, 0 here)
+        if (qi < G.rsn && hh == 0) {
+            const int64_t wrow = ((int64_t)b * P.heads + h) * G.rsn + qi;
             if (G.seeds) {
-                G.ws_D[row] = -dpi;
-                G.ws_lse[row] = lseb * (SOFTCLAMP ? kLog2e : -1.f / P.scale);
+                G.ws_D[wrow] = -dpi;
+                G.ws_lse[wrow] = lseb * (SOFTCLAMP ? kLog2e : -1.f / P.scale);
             } else {
-                G.ws_D[row] = dpi;
-                G.ws_lse[row] = lseb;
+                G.ws_D[wrow] = dpi;
+                G.ws_lse[wrow] = lseb;
             }
         }
     } else {
@@ -1034,7 +1037,8 @@ __global__ __launch_bounds__(kBwdThreads, D == 64 ? (SOFTCLAMP ? 2 : 3) : 1) voi
     const int bes = P.bias.dtype == PA_F32 ? 4 : 2;
     const float bmul = FOLD ? 1.f / P.scale : kLog2e;
     srd_t rb = {0, 0, 0, 0};
-    if (HAS_BIAS) rb = make_srd(P.bias.p + P.bias.idx(b, h, 0) * bes, (uint32_t)(P.nk * bes));
+    // (whole 16-byte chunks, the last one perhaps padding: conv_bias drops keys past the end)
+    if (HAS_BIAS) rb = make_srd(P.bias.p + P.bias.idx(b, h, 0) * bes, (uint32_t)((P.nk * bes + 15) & ~15));
     uint32_t offk[NL], offv[NL];
 #pragma unroll
     for (int n = 0; n < NL; ++n) {
@@ -1097,11 +1101,11 @@ __global__ __launch_bounds__(kBwdThreads, D == 64 ? (SOFTCLAMP ? 2 : 3) : 1) voi
     };
     // this wave's converted copy of a tile's key terms; true when every one is -inf (masked
     // keys: every probability of the tile is 0)
-    auto conv_bias = [&](int stg) __attribute__((always_inline)) -> bool {
+    auto conv_bias = [&](int stg, int j0) __attribute__((always_inline)) -> bool {
         float x;
         if (bes == 4) x = sBraw[stg][lane];
         else x = (float)reinterpret_cast<const T*>(&sBraw[stg][0])[lane];
-        const float xw = bias_class(x) == 0 ? x * bmul : -INFINITY;
+        const float xw = j0 + lane < P.nk && bias_class(x) == 0 ? x * bmul : -INFINITY;
         sBw[w][lane] = xw;
         return !__any(xw != -INFINITY);
     };
@@ -1110,11 +1114,11 @@ __global__ __launch_bounds__(kBwdThreads, D == 64 ? (SOFTCLAMP ? 2 : 3) : 1) voi
         if (HAS_BIAS) {
             // tiles of masked keys are passed through (loads and barriers only); the last
             // active tile is computed even then (its probabilities are 0)
-            bool dead = conv_bias(st);
+            bool dead = conv_bias(st, (tb + t) * BN);
             while (dead && t + 1 < nact) {
                 st = st == 2 ? 0 : st + 1;
                 enter(++t);
-                dead = conv_bias(st);
+                dead = conv_bias(st, (tb + t) * BN);
             }
         }
         const int j0 = (tb + t) * BN;
@@ -1359,8 +1363,9 @@ static bool bwd_dma_ok(const GradDev& G) {
     const int64_t qspan = std::max(P.q.sn, G.dout.sn) * ((int64_t)P.nq + 2 * kKvBQ) * 2;
     const int64_t kspan = std::max(P.k.sn, P.v.sn) * ((int64_t)P.nk + 2 * 64) * 2;
     if (!(qspan < ((int64_t)1 << 31) && kspan < ((int64_t)1 << 31))) return false;
-    // lse / D rows travel in whole 16-byte chunks
-    return P.nq % 4 == 0;
+    // lse / D rows travel in whole 16-byte chunks, whose padding rows only the dQ kernel's own
+    // preprocess writes
+    return P.nq % 4 == 0 || G.fused_pre;
 }
 
 // the direct-to-LDS dQ kernel also reads the key bias as one contiguous row of whole chunks
@@ -1372,7 +1377,7 @@ static bool bwd_dq_dma_ok(const GradDev& G) {
         const int64_t es = P.bias.dtype == PA_F32 ? 4 : 2;
         if (P.bias.sn != 1) return false;
         if ((uintptr_t)P.bias.p % 16 != 0 || (P.bias.sh * es) % 16 != 0 || (P.bias.sb * es) % 16 != 0) return false;
-        if ((P.nk * es) % 16 != 0) return false;
+        if ((P.nk * es) % 16 != 0 && !(es == 4 && (P.flags & PA_FLAG_BIAS_PADDED))) return false;
     }
     return true;
 }

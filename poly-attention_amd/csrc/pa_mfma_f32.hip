@@ -549,7 +549,7 @@ __global__ __launch_bounds__(64 * R * C, R * C / 4) void k_mfma_bwd_f32_dq(GradD
     ln.init(lane);
     const int q0 = (qb * R + wr) * 32, qi = q0 + ln.col;
     const bool qrow = qi < P.nq;
-    const int64_t r = ((int64_t)b * P.heads + h) * P.nq + (qrow ? qi : 0);
+    const int64_t r = ((int64_t)b * P.heads + h) * G.rsn + (qrow ? qi : 0);
     const float lse_l2 = qrow ? G.ws_lse[r] * kLog2e : INFINITY;
     const float dsum = qrow ? G.ws_D[r] : 0.f;
     f32x16_t dq[D / 32];
@@ -668,7 +668,7 @@ __global__ __launch_bounds__(64 * R * C, R * C / 4) void k_mfma_bwd_f32_dkv(Grad
     float rl = 0.f, rd = 0.f;
     auto load = [&](int hr, int i0) __attribute__((always_inline)) {
         const int h = h0 + hr;
-        const int64_t row0 = ((int64_t)b * P.heads + h) * P.nq;
+        const int64_t row0 = ((int64_t)b * P.heads + h) * G.rsn;
         st.load(P.q.row<float>(b, h, 0), P.q.sn, G.dout.row<float>(b, h, 0), G.dout.sn, nullptr, 0, i0,
                 P.nq);
         if (tid < C * kF32BN) {

@@ -641,7 +641,8 @@ __global__ __launch_bounds__(kFwdThreads, D == 64 ? 2 : 1) void k_mfma_fwd_dma(P
     const int bes = P.bias.dtype == PA_F32 ? 4 : 2;  // bias element size
     const float bmul = 1.f / P.scale;
     srd_t rb = {0, 0, 0, 0};
-    if (HAS_BIAS) rb = make_srd(P.bias.p + P.bias.idx(b, h, 0) * bes, (uint32_t)(P.nk * bes));
+    // (whole 16-byte chunks, the last one perhaps padding: keys past the end are dropped below)
+    if (HAS_BIAS) rb = make_srd(P.bias.p + P.bias.idx(b, h, 0) * bes, (uint32_t)((P.nk * bes + 15) & ~15));
     // per-thread byte offsets (tile-relative) of the chunks this thread loads: chunk
     // p = n*256 + tid of the tile sits at row p / CPR, physical chunk p % CPR
     uint32_t offk[NL], offv[NL];
@@ -737,7 +738,7 @@ __global__ __launch_bounds__(kFwdThreads, D == 64 ? 2 : 1) void k_mfma_fwd_dma(P
             float x;
             if (bes == 4) x = sBraw[st][lane];
             else x = (float)reinterpret_cast<const T*>(&sBraw[st][0])[lane];
-            const float xw = bias_class(x) == 0 ? x * bmul : -INFINITY;
+            const float xw = j0 + lane < P.nk && bias_class(x) == 0 ? x * bmul : -INFINITY;
             sBw[w][lane] = xw;
             // a tile whose every key term is -inf (masked keys: padding) adds nothing to any
             // row; a row that has seen only such keys keeps m = -inf and l = 0 either way
@@ -1362,7 +1363,8 @@ static bool dma_ok(const PassDev& P, int bn) {
     if (P.bias.ok()) {
         const int64_t es = P.bias.dtype == PA_F32 ? 4 : 2;
         if ((uintptr_t)P.bias.p % 16 != 0 || (P.bias.sh * es) % 16 != 0 || (P.bias.sb * es) % 16 != 0) return false;
-        if ((P.nk * es) % 16 != 0) return false;  // whole 16-byte chunks in range
+        // whole 16-byte chunks in range: of the row, or of its readable padding
+        if ((P.nk * es) % 16 != 0 && !(es == 4 && (P.flags & PA_FLAG_BIAS_PADDED))) return false;
     }
     return true;
 }

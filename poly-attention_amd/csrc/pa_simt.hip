@@ -451,7 +451,7 @@ __global__ __launch_bounds__(kSimtRows) void k_bwd_pre(GradDev G) {
         // an all -inf row (c1 == 0): its NaN output has no gradient here
         dsum = c1 > 0.f ? dsum - c1 * dl : 0.f;
     }
-    const int64_t r = ((int64_t)b * P.heads + h) * P.nq + i;
+    const int64_t r = ((int64_t)b * P.heads + h) * G.rsn + i;
     G.ws_D[r] = dsum;
     G.ws_lse[r] = lseb;
     G.ws_invc[r] = invc;
@@ -467,7 +467,7 @@ __global__ __launch_bounds__(256) void k_bwd_pre_vec(GradDev G) {
     const int h = blockIdx.y, b = blockIdx.z;
     const int sub = threadIdx.x % LPR, d0 = sub * 8;
     const int i0 = (int)blockIdx.x * kRows * kPreRows + (int)threadIdx.x / LPR;
-    const int64_t row0 = ((int64_t)b * P.heads + h) * P.nq;
+    const int64_t row0 = ((int64_t)b * P.heads + h) * G.rsn;
     // a lane group takes rows i0, i0 + kRows, ... of (b, h): every load of its rows goes out
     // before the first is used (one memory round trip per workgroup)
     uint4 ov[kPreRows], gv[kPreRows];
@@ -527,7 +527,7 @@ __global__ __launch_bounds__(kSimtRows) void k_simt_bwd_dq(GradDev G) {
     const int i = blockIdx.x * kSimtRows + threadIdx.x;
     const bool row = i < P.nq;
     const bool qok = row && P.qm.keep(b, i);
-    const int64_t r = ((int64_t)b * P.heads + h) * P.nq + (row ? i : 0);
+    const int64_t r = ((int64_t)b * P.heads + h) * G.rsn + (row ? i : 0);
     const float Dp = row ? G.ws_D[r] : 0.f;
     const float lseb = row ? G.ws_lse[r] : 0.f;
     const float invc = row ? G.ws_invc[r] : 0.f;
@@ -614,7 +614,7 @@ __global__ __launch_bounds__(kSimtRows) void k_simt_bwd_dkv(GradDev G) {
             // skipped unless one of its rows is fully masked
             for (int ii = threadIdx.x; ii < kSimtKT; ii += blockDim.x) {
                 const int i = i0 + ii;
-                const int64_t r = ((int64_t)b * P.heads + h) * P.nq + i;
+                const int64_t r = ((int64_t)b * P.heads + h) * G.rsn + i;
                 const bool ok = i < P.nq;
                 sL[ii] = ok ? G.ws_lse[r] : 0.f;
                 sI[ii] = ok ? G.ws_invc[r] : 0.f;
@@ -802,7 +802,7 @@ __global__ __launch_bounds__(256) void k_fix_rows(GradDev G) {
     static_assert(kFixRowChunk % (R * U) == 0, "whole rounds per chunk");
     const int c = blockIdx.x, h = blockIdx.y, b = blockIdx.z;
     const int slot = threadIdx.x / LPR, c0 = (threadIdx.x % LPR) * 8;
-    const int64_t row0 = ((int64_t)b * P.heads + h) * P.nq;
+    const int64_t row0 = ((int64_t)b * P.heads + h) * G.rsn;
     const int i0 = c * kFixRowChunk, i1 = min(P.nq, i0 + kFixRowChunk);
     float* part = G.ws_part + (((int64_t)b * P.heads + h) * fix_row_chunks(P.nq) + c) * (D + 2);
     bool any = false;
@@ -981,7 +981,7 @@ __global__ __launch_bounds__(kSimtRows) void k_fix_rows_b(GradDev G) {
     const int kh = h / (P.heads / G.hk);
     if (G.ws_kcnt[2 * ((int64_t)b * G.hk + kh) + 1] == 0) return;
     const int i = blockIdx.x * kSimtRows + threadIdx.x;
-    const int64_t r = ((int64_t)b * P.heads + h) * P.nq + i;
+    const int64_t r = ((int64_t)b * P.heads + h) * G.rsn + i;
     const bool dg = i < P.nq && degenerate_row(G, r) && P.qm.keep(b, i);
     if (!__syncthreads_or(dg)) return;
     const float Dp = dg ? G.ws_D[r] : 0.f;
@@ -1061,7 +1061,7 @@ __global__ __launch_bounds__(kSimtRows) void k_fix_keys_b(GradDev G) {
             if (P.causal && i0 + cnt - 1 < j_first) continue;  // every row precedes these keys
             for (int ii = threadIdx.x; ii < kSimtKT; ii += blockDim.x) {
                 const int i = i0 + ii;
-                const int64_t r = ((int64_t)b * P.heads + h) * P.nq + i;
+                const int64_t r = ((int64_t)b * P.heads + h) * G.rsn + i;
                 const bool dg = i < P.nq && degenerate_row(G, r) && P.qm.keep(b, i);
                 sL[ii] = dg ? 1.f : 0.f;
                 sI[ii] = dg ? G.ws_invc[r] : 0.f;

@@ -28,6 +28,7 @@ from . import _lib
 from ._lib import (
     DTYPE_CODE,
     PA_EPI_ROOT_SIGMOID,
+    PA_FLAG_BIAS_PADDED,
     PA_FLAG_DISCARD_OUT,
     PA_FLAG_MAY_DEGENERATE,
     PA_NORM_K,
@@ -78,6 +79,27 @@ def _empty_heads(shape, like: Tensor, dtype=None) -> Tensor:
     if _heads_inner(like):
         return torch.empty(B, N, H, d, dtype=dtype, device=like.device).permute(0, 2, 1, 3)
     return torch.empty(B, H, N, d, dtype=dtype, device=like.device)
+
+
+def _empty_lse(B: int, H: int, n: int, like: Tensor) -> Tensor:
+    """A new fp32 [B, H, n] tensor whose rows start on 16 bytes and may be read up to the next
+    multiple of four elements (PA_FLAG_BIAS_PADDED where it becomes a key bias)."""
+    pad = -n % 4
+    t = like.new_empty(B, H, n + pad, dtype=torch.float32)
+    return t[..., :n] if pad else t
+
+
+def _bias_flags(bias: Optional[Tensor]) -> int:
+    """PA_FLAG_BIAS_PADDED for an fp32 bias whose rows, of a length that is not a multiple of four,
+    lie in storage that reaches to the next multiple after every row."""
+    if bias is None or bias.shape[2] % 4 == 0 or bias.dtype != torch.float32:
+        return 0
+    B, H, n = bias.shape
+    sb, sh, sn = bias.stride()
+    if sn != 1 or sb < 0 or sh < 0:
+        return 0
+    end = bias.storage_offset() + (B - 1) * sb + (H - 1) * sh + n + (-n % 4)
+    return PA_FLAG_BIAS_PADDED if 4 * end <= bias.untyped_storage().nbytes() else 0
 
 
 def _mask(m: Optional[Tensor]) -> PaMask:
@@ -153,7 +175,7 @@ def _pass_struct(q, k, v, vmul, bias, key_mask, query_mask, out, lse, causal, so
     p.scale = float(scale)
     p.softclamp = float(softclamp) if softclamp else 0.0
     p.causal = int(bool(causal))
-    p.flags = PA_FLAG_MAY_DEGENERATE if may_degenerate else 0
+    p.flags = (PA_FLAG_MAY_DEGENERATE if may_degenerate else 0) | _bias_flags(bias)
     p.q, p.k, p.v = _view(q), _view(k), _view(v)
     p.vmul, p.bias = _view(vmul), _view(bias)
     p.key_mask, p.query_mask = _mask(key_mask), _mask(query_mask)
@@ -254,7 +276,7 @@ def _pass_prepare(q, k, v, vmul, bias, key_mask, query_mask, causal, softclamp, 
     B, _, nq, d = q.shape
     H = _pass_heads(q, k, v, vmul, bias)
     out = _empty_heads((B, H, nq, d), q)
-    lse = torch.empty(B, H, nq, dtype=torch.float32, device=q.device)
+    lse = _empty_lse(B, H, nq, q)
     y = epi = None
     if epilogue is not None:
         y = _empty_heads((B, H, nq, d), q)
@@ -385,7 +407,7 @@ def _(q, k, v, vmul, bias, key_mask, query_mask, causal, softclamp, scale, may_d
     q = _inner_contig(q)
     B, _, nq, d = q.shape
     H = _pass_heads(q, k, v, vmul, bias)
-    return (_empty_heads((B, H, nq, d), q), q.new_empty(B, H, nq, dtype=torch.float32))
+    return (_empty_heads((B, H, nq, d), q), _empty_lse(B, H, nq, q))
 
 
 @torch.library.custom_op("polyattn::pass_bwd", mutates_args=(), device_types="cuda")
