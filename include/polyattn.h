@@ -153,8 +153,9 @@ typedef struct pa_pass {
     pa_view lse;          /* [B, heads, nq], PA_F32 */
     const pa_epilogue* epi;  /* optional module epilogue (NULL: none) */
     /* Optional forward workspace of pa_attn_pass_fwd_workspace() bytes (ignored by the
-     * backward): with it a key-masked pass folds its key mask into a per-key term and takes
-     * the faster forward kernel; without it the results are the same. */
+     * backward): with it a key-masked pass folds its key mask into a per-key term, a pass with
+     * a value multiplier the product v * vmul into one tensor, and takes the faster forward
+     * kernel; without it the results are the same. */
     void*   workspace;
     size_t  workspace_bytes;
     const pa_qk_norm* norm;  /* optional q / k norms on load (NULL: none; forward only) */

@@ -179,9 +179,25 @@ int bwd_row_stride(const pa_pass& f) { return (f.nq + 3) & ~3; }
 
 size_t elem_bytes(int dtype) { return dtype == PA_F32 ? 4 : 2; }
 
+// the effective value of a 16-bit pass with a value multiplier on the direct-to-LDS kernels
+// (pa_value.hip): its head count (the values' where the multiplier has as many, else the pass's)
+// and bytes
+int value_heads(const pa_pass& f) { return f.v.heads == f.vmul.heads ? f.v.heads : f.heads; }
+
+size_t value_bytes(const pa_pass& f) {
+    if (!f.vmul.ptr || (f.q.dtype != PA_BF16 && f.q.dtype != PA_F16)) return 0;
+    if (f.dim != 64 && f.dim != 128) return 0;
+    return align256((size_t)f.batch * value_heads(f) * f.nk * f.dim * 2);
+}
+
+DView value_view(const pa_pass& f, void* p) {
+    const int64_t sh = (int64_t)f.nk * f.dim;
+    return DView{static_cast<char*>(p), sh * value_heads(f), sh, f.dim, f.heads / value_heads(f), f.q.dtype};
+}
+
 // forward workspace: the per-key term of a key-masked 16-bit pass on the MFMA kernels, whose
 // key bias it then is, and the range of keys that can enter a normal row
-size_t fwd_ws_bytes(const pa_pass& f) {
+size_t fwd_key_bytes(const pa_pass& f) {
     if (!f.key_mask.ptr || (f.q.dtype != PA_BF16 && f.q.dtype != PA_F16)) return 0;
     if (f.dim != 64 && f.dim != 128) return 0;
     if (f.bias.ptr && f.bias.heads != f.k.heads) return 0;  // one key term per key head
@@ -190,9 +206,12 @@ size_t fwd_ws_bytes(const pa_pass& f) {
            align256(kheads * 2 * sizeof(int32_t));
 }
 
+size_t fwd_ws_bytes(const pa_pass& f) { return fwd_key_bytes(f) + value_bytes(f); }
+
 // [D | lse | 1/c1] per query row; with an epilogue the gradient reaching the pass output;
 // masked passes add the key term (with a key mask), the per-head fully-masked-row sums, the
-// per-key-head bias-class counts and the per-key-head range of keys that can enter a normal row
+// per-key-head bias-class counts and the per-key-head range of keys that can enter a normal row;
+// passes with a value multiplier the effective value
 size_t bwd_ws_bytes(const pa_pass& f) {
     const size_t rows = (size_t)f.batch * f.heads * f.nq;
     size_t n = 3 * align256((size_t)f.batch * f.heads * bwd_row_stride(f) * sizeof(float));
@@ -203,7 +222,7 @@ size_t bwd_ws_bytes(const pa_pass& f) {
         n += align256((size_t)f.batch * f.heads * fix_row_chunks(f.nq) * (f.dim + 2) * sizeof(float));
         n += 2 * align256(kheads * 2 * sizeof(int32_t));
     }
-    return n;
+    return n + value_bytes(f);
 }
 
 }  // namespace
@@ -363,29 +382,39 @@ int pa_attn_pass_fwd(const pa_pass* p, void* stream) {
     const int T = p->q.dtype;
     PA_TRY(check_norm(p, P));
     if (mfma_fwd_supported(P, T)) {
+        // with its workspace (fwd_ws_bytes) the pass runs on the direct-to-LDS kernel, which has
+        // neither a key-mask path nor a value multiplier: the key mask folded into a per-key term
+        // read as the key bias, the multiplier into the values
         const size_t need = fwd_ws_bytes(*p);
+        PassDev Pm = P;
         if (need && p->workspace && p->workspace_bytes >= need) {
-            // the key mask folded into a per-key term read as the key bias (the
-            // direct-to-LDS kernel has no key-mask path); fully-masked rows as before
-            const int hk = p->k.heads, nkp = key_term_stride(*p);
             char* w = static_cast<char*>(p->workspace);
-            float* kterm = reinterpret_cast<float*>(w);
-            GradDev G = {};  // the key-term kernel reads f and hk only
-            G.f = P;
-            G.hk = hk;
-            int32_t* live = reinterpret_cast<int32_t*>(
-                w + align256((size_t)p->batch * hk * nkp * sizeof(float)));
-            launch_key_terms(G, kterm, nkp, nullptr, live, s);  // the counts serve the backward
-            PassDev Pm = P;
-            Pm.bias = DView{reinterpret_cast<char*>(kterm), (int64_t)hk * nkp, nkp, 1,
-                            p->heads / hk, PA_F32};
-            Pm.flags |= PA_FLAG_BIAS_PADDED;
-            Pm.km.p = nullptr;
-            Pm.live = live;
-            launch_mfma_fwd(Pm, T, s);
-        } else {
-            launch_mfma_fwd(P, T, s);
+            if (fwd_key_bytes(*p)) {
+                const int hk = p->k.heads, nkp = key_term_stride(*p);
+                float* kterm = reinterpret_cast<float*>(w);
+                GradDev G = {};  // the key-term kernel reads f and hk only
+                G.f = P;
+                G.hk = hk;
+                int32_t* live = reinterpret_cast<int32_t*>(
+                    w + align256((size_t)p->batch * hk * nkp * sizeof(float)));
+                launch_key_terms(G, kterm, nkp, nullptr, live, s);  // the counts serve the backward
+                Pm.bias = DView{reinterpret_cast<char*>(kterm), (int64_t)hk * nkp, nkp, 1,
+                                p->heads / hk, PA_F32};
+                Pm.flags |= PA_FLAG_BIAS_PADDED;
+                Pm.km.p = nullptr;
+                Pm.live = live;
+            }
+            if (value_bytes(*p)) {
+                PassDev Pv = Pm;
+                Pv.v = value_view(*p, w + fwd_key_bytes(*p));
+                Pv.vmul.p = nullptr;
+                if (mfma_fwd_dma_applies(Pv)) {
+                    launch_value_mul(P, Pv.v.p, value_heads(*p), T, s);
+                    Pm = Pv;
+                }
+            }
         }
+        launch_mfma_fwd(Pm, T, s);
         const bool may_degenerate = (p->flags & PA_FLAG_MAY_DEGENERATE) || p->key_mask.ptr ||
                                     p->query_mask.ptr;
         if (may_degenerate) launch_fwd_fixup(P, T, s);
@@ -503,6 +532,24 @@ int pa_attn_pass_bwd(const pa_pass_grad* g, void* stream) {
     G.seeds = 0;
     G.ws_kcnt = nullptr;
     G.ws_part = nullptr;
+    G.xv = G.xm = to_dview(none, H);
+    // the effective value at the workspace's end (value_bytes)
+    char* const vals = static_cast<char*>(g->workspace) + need - value_bytes(*p);
+    // a pass that the direct-to-LDS kernels take but for its value multiplier: folded into the
+    // values, the dK/dV kernel forming dv and dvmul
+    auto fold_value = [&](GradDev& M) {
+        if (!value_bytes(*p)) return;
+        GradDev F = M;
+        F.xv = M.f.v;
+        F.xm = M.f.vmul;
+        F.f.v = value_view(*p, vals);
+        F.f.vmul.p = nullptr;
+        F.fused_pre = mfma_bwd_fuses_pre(F) ? 1 : 0;
+        // (the kernel is built for passes with a key term, as every middle level has)
+        if (!F.f.bias.ok() || !mfma_bwd_supported(F, T) || !mfma_bwd_dma_applies(F)) return;
+        launch_value_mul(M.f, vals, value_heads(*p), T, s);
+        M = F;
+    };
     if (pass_masked(*p) && mfma_bwd_masked_supported(G, T)) {
         // normal rows on the MFMA kernels with the key mask folded into the key bias; the
         // preprocess marks fully-masked rows (lse = +inf), whose part the fix-ups add
@@ -538,12 +585,14 @@ int pa_attn_pass_bwd(const pa_pass_grad* g, void* stream) {
         // the direct-to-LDS dQ kernel does the preprocess of the normal rows where it applies
         // (fully-masked rows get lse +inf there: no normal entry; k_fix_rows does the rest of
         // their preprocess from the original masks)
+        fold_value(Gm);
         Gm.fused_pre = mfma_bwd_fuses_pre(Gm) ? 1 : 0;
         if (!Gm.fused_pre) launch_simt_bwd(G, T, s, /*pre=*/true, false, false);
         launch_mfma_bwd(Gm, T, s);
         launch_mask_fixups(G, T, s);
     } else if (mfma_bwd_supported(G, T)) {
         // the direct-to-LDS dQ kernel computes the per-row preprocess itself when it applies
+        fold_value(G);
         G.fused_pre = mfma_bwd_fuses_pre(G) ? 1 : 0;
         if (!G.fused_pre) launch_simt_bwd(G, T, s, /*pre=*/true, false, false);
         launch_mfma_bwd(G, T, s);

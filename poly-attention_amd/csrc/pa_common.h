@@ -116,6 +116,8 @@ struct GradDev {
     PassDev f;
     DView dout, dlse, dq, dk, dv, dvmul, dbias;
     DView droot, dgate;    // epilogue input gradients (with f.ey)
+    DView xv, xm;          // a value multiplier folded into f.v: the values and the multiplier, by
+                           // which the dK/dV kernel turns its gradient into dv and dvmul
     int32_t accumulate;
     int32_t hk;            // key-side head count (k, v, vmul, bias share it)
     int32_t rsn;           // row stride of the next three: nq in whole 16-byte chunks

@@ -46,6 +46,12 @@ bool mfma_order2_short_applies(const PassDev& P1, const PassDev& P2, int dtype);
 void launch_order2_short(const PassDev& P1, const PassDev& P2, int dtype, hipStream_t s);
 bool mfma_bwd_supported(const GradDev& G, int dtype);
 bool mfma_bwd_fuses_pre(const GradDev& G);
+// the direct-to-LDS forward / both direct-to-LDS backward kernels take this 16-bit pass (whose value
+// multiplier, if it had one, has been folded into its values)
+bool mfma_fwd_dma_applies(const PassDev& P);
+bool mfma_bwd_dma_applies(const GradDev& G);
+// out [batch, hv, nk, dim] = v * vmul rounded to the pass dtype (16-bit)
+void launch_value_mul(const PassDev& P, void* out, int hv, int dtype, hipStream_t s);
 void launch_mfma_bwd(const GradDev& G, int dtype, hipStream_t s);
 
 // decode

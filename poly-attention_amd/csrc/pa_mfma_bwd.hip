@@ -356,7 +356,9 @@ __device__ __forceinline__ int swz_qt(int r) {
 
 constexpr int kKvStages = 3;
 
-template <typename T, int D, bool CAUSAL, bool SOFTCLAMP, bool HAS_BIAS>
+// XV: the values are v * vmul (GradDev::xv, xm) and dv and dvmul are formed from their gradient.  A
+// template argument: as a run-time test the epilogue's registers cost every pass 3% of this kernel.
+template <typename T, int D, bool CAUSAL, bool SOFTCLAMP, bool HAS_BIAS, bool XV>
 __global__ __launch_bounds__(kBwdThreads, D == 64 ? 2 : 1) void k_mfma_bwd_dkv_dma(GradDev G) {
     using M = Mma<T>;
     typedef typename M::frag frag;
@@ -654,18 +656,48 @@ __global__ __launch_bounds__(kBwdThreads, D == 64 ? 2 : 1) void k_mfma_bwd_dkv_d
     T* dvrow = G.dv.wrow<T>(b, h0, key);
     const bool acc_k = (G.accumulate & PA_ACC_DK) != 0;
     const bool acc_v = (G.accumulate & PA_ACC_DV) != 0;
+    // the values and the multiplier of the lane's key, every word loaded before the first is used
+    u32x2_t mw[XV ? D / 32 : 1][4], vw[XV ? D / 32 : 1][4];
+    if constexpr (XV) {
+        const T* xm = G.xm.row<T>(b, h0, key);
+        const T* xv = G.xv.row<T>(b, h0, key);
+#pragma unroll
+        for (int x = 0; x < D / 32; ++x)
+#pragma unroll
+            for (int g = 0; g < 4; ++g) {
+                mw[x][g] = *reinterpret_cast<const u32x2_t*>(xm + x * 32 + 8 * g + 4 * hh);
+                vw[x][g] = *reinterpret_cast<const u32x2_t*>(xv + x * 32 + 8 * g + 4 * hh);
+            }
+    }
 #pragma unroll
     for (int x = 0; x < D / 32; ++x) {
 #pragma unroll
         for (int g = 0; g < 4; ++g) {
             const int d = x * 32 + 8 * g + 4 * hh;
+            u32x2_t pk;
+            if constexpr (XV) {
+                T* dmrow = G.dvmul.wrow<T>(b, h0, key) + d;
+                float mv[4], xm[4], xv[4];
+#pragma unroll
+                for (int w2 = 0; w2 < 2; ++w2) {
+                    unpack2<T>(mw[x][g][w2], xm[2 * w2], xm[2 * w2 + 1]);
+                    unpack2<T>(vw[x][g][w2], xv[2 * w2], xv[2 * w2 + 1]);
+                }
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    mv[r] = dv[x][4 * g + r] * xv[r] + ((G.accumulate & PA_ACC_DVMUL) ? to_f(dmrow[r]) : 0.f);
+                    dv[x][4 * g + r] *= xm[r];
+                }
+                pk[0] = pack2<T>(mv[0], mv[1]);
+                pk[1] = pack2<T>(mv[2], mv[3]);
+                *reinterpret_cast<u32x2_t*>(dmrow) = pk;
+            }
             float kv[4], vv[4];
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
                 kv[r] = dk[x][4 * g + r] * P.scale + (acc_k ? to_f(dkrow[d + r]) : 0.f);
                 vv[r] = dv[x][4 * g + r] + (acc_v ? to_f(dvrow[d + r]) : 0.f);
             }
-            u32x2_t pk;
             pk[0] = pack2<T>(kv[0], kv[1]);
             pk[1] = pack2<T>(kv[2], kv[3]);
             *reinterpret_cast<u32x2_t*>(dkrow + d) = pk;
@@ -1391,6 +1423,10 @@ bool mfma_bwd_fuses_pre(const GradDev& G) {
     return bwd_dq_dma_ok(G) && aligned_rows_host(P.out, 8);
 }
 
+bool mfma_bwd_dma_applies(const GradDev& G) {
+    return mfma_bwd_fuses_pre(G) && bwd_dma_ok(G);
+}
+
 template <typename T, int D, bool C, bool S, bool V, bool B>
 static void launch_dq(const GradDev& G, hipStream_t s) {
     const PassDev& P = G.f;
@@ -1421,7 +1457,14 @@ static void launch_bwd_t(const GradDev& G0, hipStream_t s) {
         bool done = false;
         if constexpr (D != 256) {  // head dim 256: the register-staged kernel only
             if (kv_dma) {
-                hipLaunchKernelGGL((k_mfma_bwd_dkv_dma<T, D, C, S, B>), grid, dim3(kBwdThreads), 0, s, G);
+                if constexpr (B) {
+                    if (G.xm.ok()) {
+                        hipLaunchKernelGGL((k_mfma_bwd_dkv_dma<T, D, C, S, B, true>), grid, dim3(kBwdThreads), 0, s, G);
+                        done = true;
+                    }
+                }
+                if (!done)
+                    hipLaunchKernelGGL((k_mfma_bwd_dkv_dma<T, D, C, S, B, false>), grid, dim3(kBwdThreads), 0, s, G);
                 done = true;
             }
         }

@@ -1369,6 +1369,9 @@ static bool dma_ok(const PassDev& P, int bn) {
     return true;
 }
 
+bool mfma_fwd_dma_applies(const PassDev& P) {
+    return (P.dim == 64 || P.dim == 128) && !P.vmul.ok() && dma_ok(P, 64);
+}
 
 // ---------------------------------------------------------------------------------------
 

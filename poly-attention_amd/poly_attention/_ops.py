@@ -288,7 +288,7 @@ def _pass_prepare(q, k, v, vmul, bias, key_mask, query_mask, causal, softclamp, 
         norm = _qk_norm_struct(qk_norm)
         p.norm = ctypes.addressof(norm)
     ws = None
-    if km is not None:  # a key-masked pass takes the faster kernel with a workspace
+    if km is not None or vmul is not None:  # such a pass takes the faster kernel with a workspace
         ws_bytes = lib.pa_attn_pass_fwd_workspace(ctypes.byref(p))
         if ws_bytes:
             ws = torch.empty(ws_bytes, dtype=torch.uint8, device=q.device)
