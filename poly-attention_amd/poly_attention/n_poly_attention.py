@@ -30,8 +30,8 @@ from ._helpers import (
     where_keys,
     where_queries,
 )
-from .poly_attention import (_DECODE_ROWS, _compute_dtype, _q_norms, _static_decode_step,
-                             fused_available)
+from .poly_attention import (_DECODE_ROWS, _compute_dtype, _module_angles, _q_norms,
+                             _static_decode_step, fused_available)
 from .rotary import RotaryEmbedding, apply_rotary_emb
 
 LinearNoBias = partial(nn.Linear, bias=False)
@@ -225,7 +225,14 @@ class NPolyAttention(Module):
                 root_value = repeat_kv(root_value, self.num_rep)
         else:
             # the q norms and the external rotary (fused into one kernel on the GPU path)
-            qs = _q_norms(self, self.q_norms, qs, rotary_pos_emb)
+            # or the module's own where it can go with the norms; a returned cache holds the keys
+            # unrotated
+            angles = _module_angles(self, qs, rotary_pos_emb, cache)
+            rotated = _q_norms(self, self.q_norms, qs, angles) if exists(angles) else None
+            if not exists(rotated) or return_cache:
+                qs = _q_norms(self, self.q_norms, qs, rotary_pos_emb)
+            else:
+                qs = rotated
 
             q1 = first(qs)
             qs_rest = qs[1:]
@@ -233,7 +240,7 @@ class NPolyAttention(Module):
             if self._use_fused(q1):
                 out, new_cache = self._fused_core(q1, qs_rest, vs_for_aggregation, mask,
                                                   context_mask, rotary_pos_emb, cache,
-                                                  return_cache, epilogue)
+                                                  return_cache, epilogue, rotated)
                 epilogue_done = True
             else:
                 out, new_cache, root_value = self._eager_core(q1, qs_rest, vs_for_aggregation,
@@ -342,9 +349,10 @@ class NPolyAttention(Module):
         return out, new_cache, root_value
 
     def _fused_core(self, q1, qs_rest, vs, mask, context_mask, rotary_pos_emb, cache,
-                    return_cache, epilogue):
+                    return_cache, epilogue, rotated=None):
         """The order-n chain on the HIP kernels (qs_rest / vs stay at kv_heads), with the
-        module epilogue applied: fused into the final pass on the order-2 chain's path."""
+        module epilogue applied: fused into the final pass on the order-2 chain's path.
+        ``rotated``: (q1, ..., q_{order+1}) with the module's own rotary applied (no cache)."""
         from . import _ops
 
         order = self.order
@@ -357,7 +365,10 @@ class NPolyAttention(Module):
 
         if not exists(cache):
             q_left, q_right = [q1, *qs_rest[:-1]], list(qs_rest)
-            if module_rotary:
+            if exists(rotated):
+                rotated = [t.to(dt) for t in rotated]
+                q_left, q_right = rotated[:-1], rotated[1:]
+            elif module_rotary:
                 rotated = [self.rotary_emb.rotate_queries_with_cached_keys(ql, qr)
                            for ql, qr in zip(q_left, q_right)]
                 q_left, q_right = (list(t) for t in zip(*rotated))

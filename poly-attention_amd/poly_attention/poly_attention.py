@@ -73,6 +73,34 @@ def _q_norms(module, norms, qs, rotary_pos_emb=None):
     return tuple(out)
 
 
+def _module_angles(module, qs, rotary_pos_emb, cache):
+    """The rotary angles of the module's own rotary embedding (poly_attention.py:302-304,
+    n_poly_attention.py:224-229) for ``qs`` = (q1, ..., q_{order+1}) of one length without a cache,
+    where the q norms can apply them (pa_rmsnorm's rotation, the rounding of
+    apply_rotary_emb): every left and right query of a pass then has the positions 0 .. n - 1.
+    None where the rotation stays with the rotary module: an external rotary, a cache, other
+    lengths, learned frequencies, norms that pa_rmsnorm does not take, under torch.compile."""
+    rot = module.rotary_emb
+    if exists(rotary_pos_emb) or exists(cache) or type(rot) is not RotaryEmbedding:
+        return None
+    q0 = qs[0]
+    if (torch.compiler.is_compiling() or rot.freqs.requires_grad or not module._use_fused(q0)
+            or rot._forward_hooks or rot._forward_pre_hooks or torch.is_autocast_enabled("cuda")):
+        return None
+    from . import _ops
+
+    if any(q.shape[-2] != q0.shape[-2] or q.dtype != q0.dtype for q in qs):
+        return None
+    if not all(type(n) is RMSNorm and tuple(n.normalized_shape) == (q.shape[-1],)
+               and (n.weight is None or n.weight.dtype == q.dtype) for n, q in zip(module.q_norms, qs)):
+        return None
+    with torch.no_grad():
+        angles = rot(rot.get_seq_pos(q0.shape[-2], device=q0.device, dtype=q0.dtype))
+    if not all(_ops.rms_supported(q, n.weight, angles) for n, q in zip(module.q_norms, qs)):
+        return None
+    return angles
+
+
 def _q_norms_one_launch(module, norms, qs, rotary_pos_emb):
     """The norms of ``qs`` in one pa_rmsnorm_fwd_many launch when that applies: the fused GPU
     path, no gradient, no rotary, not under torch.compile, every norm an RMSNorm over the
@@ -424,8 +452,17 @@ class Order2PolyAttention(Module):
             # the norms applied by the attention passes as they load q1 / q2 / q3
             norms_on_load = self._norms_on_load(qs, v3, mask, context_mask, rotary_pos_emb,
                                                 cache, return_cache)
+            rotated = None
             if norms_on_load is None:
-                qs = _q_norms(self, self.q_norms, qs, rotary_pos_emb)
+                # the module's own rotary goes with the norms where it can; a returned cache holds
+                # the keys unrotated
+                angles = _module_angles(self, qs, rotary_pos_emb, cache)
+                if exists(angles):
+                    rotated = _q_norms(self, self.q_norms, qs, angles)
+                if not exists(rotated) or return_cache:
+                    qs = _q_norms(self, self.q_norms, qs, rotary_pos_emb)
+                else:
+                    qs = rotated
 
             q1, q2, q3 = qs
 
@@ -439,7 +476,7 @@ class Order2PolyAttention(Module):
             if self._use_fused(q1):
                 out, new_cache = self._fused_core(q1, q2, q3, v3, mask, context_mask,
                                                   rotary_pos_emb, cache, return_cache, epilogue,
-                                                  norms_on_load)
+                                                  norms_on_load, rotated)
                 epilogue_done = True
             else:
                 out, new_cache, v2 = self._eager_core(q1, q2, q3, v2, v3, mask, context_mask,
@@ -526,10 +563,11 @@ class Order2PolyAttention(Module):
                      for w, n in zip(weights, norms))
 
     def _fused_core(self, q1, q2, q3, v3, mask, context_mask, rotary_pos_emb, cache,
-                    return_cache, epilogue, qk_norms=None):
+                    return_cache, epilogue, qk_norms=None, rotated=None):
         """The attention core on the HIP kernels (q2 / q3 / v3 stay at kv_heads), with the
         module epilogue applied: fused into pass 2 on the order-2 chain's path.  ``qk_norms``:
-        q1 / q2 / q3 are not normalised yet and the passes apply these norms on load."""
+        q1 / q2 / q3 are not normalised yet and the passes apply these norms on load.
+        ``rotated``: q1 / q2 / q3 with the module's own rotary applied (no cache)."""
         from . import _ops
 
         rep = self.num_rep if self.is_gqa else 1
@@ -539,7 +577,10 @@ class Order2PolyAttention(Module):
 
         if not exists(cache):
             q1r, q2r_right, q2r_left, q3r = q1, q2, q2, q3
-            if module_rotary:
+            if exists(rotated):
+                q1r, q2r_right, q3r = (t.to(dt) for t in rotated)
+                q2r_left = q2r_right
+            elif module_rotary:
                 q1r, q2r_right = self.rotary_emb.rotate_queries_with_cached_keys(q1, q2)
                 q2r_left, q3r = self.rotary_emb.rotate_queries_with_cached_keys(q2, q3)
             out, lses, msgs = _ops.poly_chain(
