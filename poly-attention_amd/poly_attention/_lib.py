@@ -8,6 +8,7 @@ from __future__ import annotations
 
 import ctypes
 import os
+import struct
 from ctypes import c_float, c_int, c_int32, c_int64, c_size_t, c_void_p
 from pathlib import Path
 
@@ -263,6 +264,19 @@ class PaKernelTime(ctypes.Structure):
 
 STRUCTS = (PaView, PaMask, PaPass, PaPassGrad, PaDecodeLevel, PaDecode, PaPrologueItem,
            PaPrologue, PaRmsNorm, PaLinear, PaLinearOut, PaEpilogue, PaQkNorm)
+
+
+# The hot structs as one struct.pack each (assigning ctypes fields one by one was half of a pass's
+# host time): a view is (ptr, sb, sh, sn, heads, dtype), a mask (ptr, sb, sn).
+_VIEW_FMT = "Q3q2i"
+NO_VIEW = (0, 0, 0, 0, 0, 0)
+NO_MASK = (0, 0, 0)
+_PASS_FMT = "5i2f2i4x" + 5 * _VIEW_FMT + 2 * "Q2q" + 2 * _VIEW_FMT + "4Q"
+PACK_PASS = struct.Struct("@" + _PASS_FMT)
+PACK_PASS_GRAD = struct.Struct("@" + _PASS_FMT + 7 * _VIEW_FMT + "i4x2Q" + 2 * _VIEW_FMT)
+PACK_RMS = struct.Struct("@4if4x" + _VIEW_FMT + "Qi4x" + _VIEW_FMT + "Q" + 2 * _VIEW_FMT + "4Q2iq")
+for _pack, _cls in ((PACK_PASS, PaPass), (PACK_PASS_GRAD, PaPassGrad), (PACK_RMS, PaRmsNorm)):
+    assert _pack.size == ctypes.sizeof(_cls), _cls.__name__
 
 
 class PolyAttnError(RuntimeError):

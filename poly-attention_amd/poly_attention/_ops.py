@@ -17,7 +17,6 @@
 
 from __future__ import annotations
 
-import contextlib
 import ctypes
 from typing import Optional, Sequence
 
@@ -35,7 +34,6 @@ from ._lib import (
     PA_NORM_Q,
     PaDecode,
     PaEpilogue,
-    PaMask,
     PaPass,
     PaPassGrad,
     PaQkNorm,
@@ -63,6 +61,21 @@ def _view(t: Optional[Tensor]) -> PaView:
     v.heads = t.shape[1]
     v.dtype = DTYPE_CODE[t.dtype]
     return v
+
+
+def _vt(t: Optional[Tensor]) -> tuple:
+    """The fields of _view(t), for the packed structs (a feature stride of 1 is the caller's)."""
+    if t is None:
+        return _lib.NO_VIEW
+    st = t.stride()
+    return (t.data_ptr(), st[0], st[1], st[2], t.shape[1], DTYPE_CODE[t.dtype])
+
+
+def _mt(m: Optional[Tensor]) -> tuple:
+    if m is None:
+        return _lib.NO_MASK
+    assert m.dtype == torch.uint8 and m.dim() == 2
+    return (m.data_ptr(), *m.stride())
 
 
 def _heads_inner(t: Tensor) -> bool:
@@ -102,31 +115,20 @@ def _bias_flags(bias: Optional[Tensor]) -> int:
     return PA_FLAG_BIAS_PADDED if 4 * end <= bias.untyped_storage().nbytes() else 0
 
 
-def _mask(m: Optional[Tensor]) -> PaMask:
-    pm = PaMask()
-    if m is None:
-        return pm
-    assert m.dtype == torch.uint8 and m.dim() == 2
-    pm.ptr = m.data_ptr()
-    pm.sb, pm.sn = m.stride(0), m.stride(1)
-    return pm
-
-
 def _mask_u8(m: Optional[Tensor]) -> Optional[Tensor]:
     if m is None:
         return None
-    return m.to(torch.uint8)
+    return m.view(torch.uint8) if m.dtype == torch.bool else m.to(torch.uint8)
 
 
-def _device(t: Tensor):
-    """The tensor's device as the current one (a no-op context when it already is)."""
-    if t.device.index is None or t.device.index == torch.cuda.current_device():
-        return contextlib.nullcontext()
-    return torch.cuda.device(t.device)
-
-
-def _stream(t: Tensor) -> int:
-    return torch.cuda.current_stream(t.device).cuda_stream
+def _call(fn, t: Tensor, what: str, *args) -> None:
+    """fn(*args, stream) on t's device and its current stream; raises on a failure status."""
+    index = t.device.index
+    if index == torch._C._cuda_getDevice():
+        _lib.check(fn(*args, torch._C._cuda_getCurrentRawStream(index)), what)
+    else:
+        with torch.cuda.device(index):
+            _lib.check(fn(*args, torch._C._cuda_getCurrentRawStream(index)), what)
 
 
 def _epilogue_struct(epilogue, y) -> PaEpilogue:
@@ -167,21 +169,20 @@ def qk_norms_fusable(q1: Tensor, q2: Tensor, q3: Tensor, v3: Tensor, weights, ca
                and w.data_ptr() % 16 == 0 for w in weights)
 
 
-def _pass_struct(q, k, v, vmul, bias, key_mask, query_mask, out, lse, causal, softclamp, scale,
-                 may_degenerate, epi: Optional[PaEpilogue] = None) -> PaPass:
-    p = PaPass()
-    p.batch, p.heads, p.nq, p.dim = q.shape[0], out.shape[1], q.shape[2], q.shape[3]
-    p.nk = k.shape[2]
-    p.scale = float(scale)
-    p.softclamp = float(softclamp) if softclamp else 0.0
-    p.causal = int(bool(causal))
-    p.flags = (PA_FLAG_MAY_DEGENERATE if may_degenerate else 0) | _bias_flags(bias)
-    p.q, p.k, p.v = _view(q), _view(k), _view(v)
-    p.vmul, p.bias = _view(vmul), _view(bias)
-    p.key_mask, p.query_mask = _mask(key_mask), _mask(query_mask)
-    p.out, p.lse = _view(out), _view(lse)
-    p.epi = ctypes.addressof(epi) if epi is not None else None
-    return p
+def _pass_fields(q, k, v, vmul, bias, key_mask, query_mask, out, lse, causal, softclamp, scale,
+                 may_degenerate, epi: Optional[PaEpilogue] = None) -> tuple:
+    """The fields of a PaPass in the order of _lib.PACK_PASS."""
+    for t in (q, k, v, out):
+        assert t.dim() == 4 and (t.stride(-1) == 1 or t.shape[-1] == 1), "feature stride must be 1"
+    B, _, nq, d = q.shape
+    return (B, out.shape[1], nq, k.shape[2], d, scale, softclamp or 0.0, bool(causal),
+            (PA_FLAG_MAY_DEGENERATE if may_degenerate else 0) | _bias_flags(bias),
+            *_vt(q), *_vt(k), *_vt(v), *_vt(vmul), *_vt(bias), *_mt(key_mask), *_mt(query_mask),
+            *_vt(out), *_vt(lse), ctypes.addressof(epi) if epi is not None else 0, 0, 0, 0)
+
+
+def _pass_struct(*args, **kw) -> PaPass:
+    return PaPass.from_buffer_copy(_lib.PACK_PASS.pack(*_pass_fields(*args, **kw)))
 
 
 def _pass_heads(q, k, v, vmul, bias) -> int:
@@ -258,8 +259,7 @@ def pass_fwd_raw(q, k, v, vmul, bias, key_mask, query_mask, causal, softclamp, s
         return tuple(t if i == 1 else _unpad(t, d, q) for i, t in enumerate(res))
     p, res, _keep = _pass_prepare(q, k, v, vmul, bias, key_mask, query_mask, causal, softclamp,
                                   scale, may_degenerate, epilogue, qk_norm)
-    with _device(q):
-        _lib.check(_lib.load().pa_attn_pass_fwd(ctypes.byref(p), _stream(q)), "pa_attn_pass_fwd")
+    _call(_lib.load().pa_attn_pass_fwd, q, "pa_attn_pass_fwd", ctypes.byref(p))
     return res
 
 
@@ -362,26 +362,24 @@ def pass_bwd_raw(dout, dlse, q, k, v, vmul, bias, key_mask, query_mask, out, lse
     dbias = (torch.empty(bias.shape, dtype=torch.float32, device=q.device)
              if bias is not None else None)
     dlse32 = dlse.float() if dlse is not None else None
-    g = PaPassGrad()
-    g.fwd = _pass_struct(q, k, v, vmul, bias, km, qm, out, lse, causal, softclamp, scale,
-                         may_degenerate or km is not None or qm is not None)
-    g.dout, g.dlse = _view(dout), _view(dlse32)
-    g.dq, g.dk, g.dv = _view(dq), _view(dk), _view(dv)
-    g.dvmul, g.dbias = _view(dvmul), _view(dbias)
-    g.accumulate = accumulate
     droot = dgate = epi = None
     if epilogue is not None:
         root, gate, _ = epilogue
         droot = _empty_heads(root.shape, root) if root is not None else None
         dgate = _empty_heads(gate.shape, gate) if gate is not None else None
         epi = _epilogue_struct(epilogue, out)  # y is not read by the backward
-        g.fwd.epi = ctypes.addressof(epi)
-        g.droot, g.dgate = _view(droot), _view(dgate)
-    ws_bytes = lib.pa_attn_pass_bwd_workspace(ctypes.byref(g))
+    for t in (dout, dq, dk, dv, dvmul):
+        assert t is None or t.stride(-1) == 1 or t.shape[-1] == 1, "feature stride must be 1"
+    g = PaPassGrad.from_buffer_copy(_lib.PACK_PASS_GRAD.pack(
+        *_pass_fields(q, k, v, vmul, bias, km, qm, out, lse, causal, softclamp, scale,
+                      may_degenerate or km is not None or qm is not None, epi),
+        *_vt(dout), *_vt(dlse32), *_vt(dq), *_vt(dk), *_vt(dv), *_vt(dvmul), *_vt(dbias), accumulate,
+        0, 0, *_vt(droot), *_vt(dgate)))
+    ref = ctypes.byref(g)
+    ws_bytes = lib.pa_attn_pass_bwd_workspace(ref)
     ws = torch.empty(max(ws_bytes, 1), dtype=torch.uint8, device=q.device)
     g.workspace, g.workspace_bytes = ws.data_ptr(), ws_bytes
-    with _device(q):
-        _lib.check(lib.pa_attn_pass_bwd(ctypes.byref(g), _stream(q)), "pa_attn_pass_bwd")
+    _call(lib.pa_attn_pass_bwd, q, "pa_attn_pass_bwd", ref)
     if dbias is not None and bias is not None and dbias.dtype != bias.dtype:
         dbias = dbias.to(bias.dtype)
     if epilogue is not None:
@@ -452,7 +450,7 @@ def _pass_setup(ctx, inputs, output):
     ctx.set_materialize_grads(False)
 
 
-def _pass_backward(ctx, dout, dlse):
+def _pass_backward(ctx, dout, dlse, raw=False):
     q, k, v, vmul, bias, key_mask, query_mask, out, lse = ctx.saved_tensors
     if dout is None:
         dout = torch.zeros_like(out)
@@ -461,7 +459,7 @@ def _pass_backward(ctx, dout, dlse):
     outs = [claim_slot(r, t) for r, t in zip(ctx.slots, (q, k, v))]
     if q.shape[1] != out.shape[1]:
         outs[0] = None
-    if any(o is not None for o in outs):
+    if raw or any(o is not None for o in outs):
         dq, dk, dv, dvmul, dbias = pass_bwd_raw(dout, dlse, q, k, v, vmul, bias, key_mask,
                                                 query_mask, out, lse, ctx.causal, ctx.softclamp,
                                                 ctx.scale, ctx.may_degenerate, dq_out=outs[0],
@@ -483,6 +481,49 @@ def _pass_backward(ctx, dout, dlse):
 torch.library.register_autograd("polyattn::pass_fwd", _pass_backward, setup_context=_pass_setup)
 
 
+def _plain_eager(*ts) -> bool:
+    """Plain eager tensors with no transform, mode or subclass that has to see the registered custom
+    op (torch.func, vmap, dispatch modes such as fake tensors, torch.compile): the call may then
+    be an autograd node of its own, whose host time is a fraction of a custom op's."""
+    return (not torch.compiler.is_compiling()
+            and torch._C._functorch.peek_interpreter_stack() is None
+            and torch._C._len_torch_dispatch_stack() == 0
+            and all(t is None or type(t) in _PLAIN for t in ts))
+
+
+_PLAIN = (Tensor, torch.nn.Parameter)
+
+
+class _PassNode(torch.autograd.Function):
+    """polyattn::pass_fwd and its backward as one autograd node (``_plain_eager`` calls)."""
+
+    @staticmethod
+    def forward(ctx, *inputs):
+        output = pass_fwd_raw(*inputs)
+        _pass_setup(ctx, inputs, output)
+        return output
+
+    @staticmethod
+    @torch.autograd.function.once_differentiable
+    def backward(ctx, dout, dlse):
+        return _pass_backward(ctx, dout, dlse, raw=True)
+
+
+class _RmsNode(torch.autograd.Function):
+    """polyattn::rms_norm and its backward as one autograd node (``_plain_eager`` calls)."""
+
+    @staticmethod
+    def forward(ctx, x, weight, eps, angles):
+        output = _rms_fwd_raw(x, weight, eps, angles)
+        _rms_setup(ctx, (x, weight, eps, angles), output)
+        return output[0]
+
+    @staticmethod
+    @torch.autograd.function.once_differentiable
+    def backward(ctx, dy):
+        return _rms_backward(ctx, dy, None, raw=True)
+
+
 def _needs_op(*ts) -> bool:
     """Whether a call must go through the registered custom op (autograd or torch.compile
     tracing); plain inference calls the library directly (less host overhead per launch)."""
@@ -501,8 +542,9 @@ def attn_pass(q: Tensor, k: Tensor, v: Tensor, vmul: Optional[Tensor] = None,
     if not _needs_op(q, k, v, vmul, bias):
         return pass_fwd_raw(q, k, v, vmul, bias, key_mask, query_mask, bool(causal),
                             float(softclamp or 0.0), float(scale), bool(may_degenerate))
-    return pass_fwd_op(q, k, v, vmul, bias, key_mask, query_mask, bool(causal),
-                       float(softclamp or 0.0), float(scale), bool(may_degenerate))
+    op = _PassNode.apply if _plain_eager(q, k, v, vmul, bias) else pass_fwd_op
+    return op(q, k, v, vmul, bias, key_mask, query_mask, bool(causal), float(softclamp or 0.0),
+              float(scale), bool(may_degenerate))
 
 
 # ---------------------------------------------------------------------------------------
@@ -519,20 +561,19 @@ def _rms_angles(x: Tensor, angles: Optional[Tensor]) -> Optional[Tensor]:
     return angles
 
 
-def _rms_struct(x: Tensor, weight: Optional[Tensor], eps: float,
-                angles: Optional[Tensor] = None) -> PaRmsNorm:
-    r = PaRmsNorm()
-    r.batch, r.heads, r.n, r.dim = x.shape
-    r.eps = float(eps)
-    r.x = _view(x)
-    if weight is not None:
-        r.weight, r.weight_dtype = weight.data_ptr(), DTYPE_CODE[weight.dtype]
+def _rms_struct(x: Tensor, weight: Optional[Tensor], eps: float, angles: Optional[Tensor] = None,
+                y: Optional[Tensor] = None, rstd: Optional[Tensor] = None,
+                dy: Optional[Tensor] = None, dx: Optional[Tensor] = None,
+                dweight: Optional[Tensor] = None) -> PaRmsNorm:
+    B, H, n, d = x.shape
     a = _rms_angles(x, angles)
-    if a is not None:
-        r.angles, r.angles_dtype = a.data_ptr(), DTYPE_CODE[a.dtype]
-        r.rot_dim = a.shape[-1]
-        r.angles_stride = a.stride(0) if a.dim() == 2 else 0
-    return r
+    rot = (0, 0, 0, 0) if a is None else (a.data_ptr(), DTYPE_CODE[a.dtype], a.shape[-1],
+                                          a.stride(0) if a.dim() == 2 else 0)
+    return PaRmsNorm.from_buffer_copy(_lib.PACK_RMS.pack(
+        B, H, n, d, eps, *_vt(x), weight.data_ptr() if weight is not None else 0,
+        DTYPE_CODE[weight.dtype] if weight is not None else 0, *_vt(y),
+        rstd.data_ptr() if rstd is not None else 0, *_vt(dy), *_vt(dx),
+        dweight.data_ptr() if dweight is not None else 0, 0, 0, *rot))
 
 
 def _aligned16(t: Tensor) -> Tensor:
@@ -583,10 +624,9 @@ def _rms_fwd_raw(x: Tensor, weight: Optional[Tensor], eps: float,
     lib = _lib.load()
     y = _empty_heads(x.shape, x)
     rstd = torch.empty(x.shape[:3], dtype=torch.float32, device=x.device)
-    r = _rms_struct(_aligned16(x), weight, eps, angles)
-    r.y, r.rstd = _view(y), rstd.data_ptr()
-    with _device(x):
-        _lib.check(lib.pa_rmsnorm_fwd(ctypes.byref(r), _stream(x)), "pa_rmsnorm_fwd")
+    x = _aligned16(x)
+    r = _rms_struct(x, weight, eps, angles, y=y, rstd=rstd)
+    _call(lib.pa_rmsnorm_fwd, x, "pa_rmsnorm_fwd", ctypes.byref(r))
     return y, rstd
 
 
@@ -612,18 +652,16 @@ def _rms_bwd_raw(dy: Tensor, x: Tensor, weight: Optional[Tensor], rstd: Tensor, 
     dx = _empty_heads(x.shape, x) if dx_out is None else dx_out
     if dx_out is not None and (not rms_supported(dx_out, weight, angles) or dx_out.data_ptr() % 16):
         dx = _empty_heads(x.shape, x)
-    r = _rms_struct(_aligned16(x), weight, eps, angles)
-    r.rstd = rstd.data_ptr()
-    r.dy, r.dx = _view(dy), _view(dx)
+    xa = _aligned16(x)
     dw32 = None
     if weight is not None:
         dw32 = torch.empty(x.shape[-1], dtype=torch.float32, device=x.device)
-        r.dweight = dw32.data_ptr()
-    ws_bytes = lib.pa_rmsnorm_bwd_workspace(ctypes.byref(r))
+    r = _rms_struct(xa, weight, eps, angles, rstd=rstd, dy=dy, dx=dx, dweight=dw32)
+    ref = ctypes.byref(r)
+    ws_bytes = lib.pa_rmsnorm_bwd_workspace(ref)
     ws = torch.empty(max(ws_bytes, 1), dtype=torch.uint8, device=x.device)
     r.workspace, r.workspace_bytes = ws.data_ptr(), ws_bytes
-    with _device(x):
-        _lib.check(lib.pa_rmsnorm_bwd(ctypes.byref(r), _stream(x)), "pa_rmsnorm_bwd")
+    _call(lib.pa_rmsnorm_bwd, x, "pa_rmsnorm_bwd", ref)
     dw = dw32.to(weight.dtype) if weight is not None else x.new_empty(0)
     return dx, dw
 
@@ -643,12 +681,12 @@ def _rms_setup(ctx, inputs, output):
     ctx.set_materialize_grads(False)
 
 
-def _rms_backward(ctx, dy, drstd):
+def _rms_backward(ctx, dy, drstd, raw=False):
     x, weight, rstd, angles = ctx.saved_tensors
     if dy is None:
         return None, None, None, None
     dx_out = claim_slot(ctx.slot, x)
-    if dx_out is not None:  # eager: write dx into the split projection's gradient
+    if raw or dx_out is not None:  # eager: dx goes into the split projection's gradient if it can
         dx, dw = _rms_bwd_raw(dy, x, weight, rstd, ctx.eps, angles, dx_out)
     else:
         dx, dw = rms_norm_bwd_op(dy, x, weight, rstd, ctx.eps, angles)
@@ -667,6 +705,8 @@ def rms_norm(x: Tensor, weight: Optional[Tensor], eps: Optional[float],
         eps = torch.finfo(torch.float32).eps
     if not _needs_op(x, weight):
         return _rms_fwd_raw(x, weight, float(eps), angles)[0]
+    if _plain_eager(x, weight):
+        return _RmsNode.apply(x, weight, float(eps), angles)
     return rms_norm_op(x, weight, float(eps), angles)[0]
 
 
@@ -683,13 +723,11 @@ def rms_norm_many(xs: Sequence[Tensor], weights: Sequence[Optional[Tensor]],
     for k, (x, w, e) in enumerate(zip(xs, weights, eps)):
         x = _aligned16(x)
         y = _empty_heads(x.shape, x)
-        r = _rms_struct(x, w, torch.finfo(torch.float32).eps if e is None else float(e))
-        r.y = _view(y)  # no rstd: nothing runs backward through these norms
-        items[k] = r
+        # (no rstd: nothing runs backward through these norms)
+        items[k] = _rms_struct(x, w, torch.finfo(torch.float32).eps if e is None else float(e), y=y)
         ys.append(y)
         keep.append(x)
-    with _device(xs[0]):
-        _lib.check(lib.pa_rmsnorm_fwd_many(items, n, _stream(xs[0])), "pa_rmsnorm_fwd_many")
+    _call(lib.pa_rmsnorm_fwd_many, xs[0], "pa_rmsnorm_fwd_many", items, n)
     return ys
 
 
@@ -779,8 +817,7 @@ def linear_small_group(x: Tensor, specs, *, x_add: Optional[Tensor] = None,
             o.residual, o.residual_stride = r2.data_ptr(), r2.stride(0)
         o.y, o.y_stride = y.data_ptr(), y.stride(0)
         outs.append(y.reshape(*x.shape[:-1], n))
-    with _device(x):
-        _lib.check(lib.pa_linear_small(ctypes.byref(lin), _stream(x)), "pa_linear_small")
+    _call(lib.pa_linear_small, x, "pa_linear_small", ctypes.byref(lin))
     if return_sum:
         return outs, xs.reshape(x.shape)
     return outs
@@ -843,6 +880,14 @@ def linear_many(layers, xs) -> list[Tensor]:
 # head split of the training / prefill projections
 
 
+def _head_view(t: Tensor, off: int, h: int, d: int) -> Tensor:
+    """t[..., off:off + h*d].unflatten(-1, (h, d)).transpose(1, 2) of a [B, N, F] tensor, in one
+    view operation."""
+    B, n, _ = t.shape
+    sb, sn, sf = t.stride()
+    return t.as_strided((B, h, n, d), (sb, d * sf, sn, sf), t.storage_offset() + off * sf)
+
+
 class _GradSlots:
     """The gradient buffer of a head-split projection ([B, N, F]), allocated on first use in the
     backward.  A backward that produces the gradient of a piece (the pass and RMSNorm
@@ -862,8 +907,7 @@ class _GradSlots:
     def view(self, i: int) -> Tensor:
         if self.buf is None:
             self.buf = torch.empty(self.shape, dtype=self.dtype, device=self.device)
-        o, h = self.offsets[i], self.heads[i]
-        return self.buf[..., o:o + h * self.d].unflatten(-1, (h, self.d)).transpose(1, 2)
+        return _head_view(self.buf, self.offsets[i], self.heads[i], self.d)
 
     def claim(self, i: int) -> Optional[Tensor]:
         if i in self.claimed:
@@ -910,7 +954,7 @@ class _SplitHeads(torch.autograd.Function):
         ctx.set_materialize_grads(False)
         outs, off = [], 0
         for h in heads:
-            outs.append(t[..., off:off + h * d].unflatten(-1, (h, d)).transpose(1, 2))
+            outs.append(_head_view(t, off, h, d))
             off += h * d
         return tuple(outs)
 
@@ -1062,9 +1106,11 @@ def project_heads(layers, xs, splits):
 def _split_heads(t: Tensor, heads, d: int):
     if not (torch.is_grad_enabled() and t.requires_grad) or torch.compiler.is_compiling():
         # no gradient (or traced): plain views, without the gradient-slot autograd node
+        plain = _plain_eager(t)
         outs, off = [], 0
         for h in heads:
-            outs.append(t[..., off:off + h * d].unflatten(-1, (h, d)).transpose(1, 2))
+            outs.append(_head_view(t, off, h, d) if plain else
+                        t[..., off:off + h * d].unflatten(-1, (h, d)).transpose(1, 2))
             off += h * d
         return tuple(outs)
     slots = _GradSlots(t.shape, t.dtype, t.device, tuple(heads), d)
@@ -1101,9 +1147,7 @@ def order2_forward(q1, q2, q3, v3, key_mask, causal, softclamp, scale, epilogue=
             qk_norm=(n1, n2) if norms is not None else None)
         if not keep_inner:
             p1.flags |= PA_FLAG_DISCARD_OUT
-        with _device(q2):
-            _lib.check(_lib.load().pa_poly_order2_fwd(ctypes.byref(p1), ctypes.byref(p2),
-                                                      _stream(q2)), "pa_poly_order2_fwd")
+        _call(_lib.load().pa_poly_order2_fwd, q2, "pa_poly_order2_fwd", ctypes.byref(p1), ctypes.byref(p2))
         return (res[0], res[1], lse23, msg) + tuple(res[2:])
     msg, lse23 = pass_fwd_raw(q2, q3, v3, None, None, key_mask, None, causal, softclamp, scale,
                               degenerate, qk_norm=(n2, n3) if norms is not None else None)
@@ -1368,15 +1412,12 @@ def poly_decode_step(q_new: Sequence[Tensor], k_caches: Sequence[Tensor],
         assert n_dev.dtype == torch.int32 and n_dev.is_cuda and n_dev.numel() == 1
         D.n_dev = n_dev.data_ptr()
     if noalloc:
-        with _device(out):
-            _lib.check(lib.pa_poly_decode_noalloc(ctypes.byref(D), _stream(out)),
-                       "pa_poly_decode_noalloc")
+        _call(lib.pa_poly_decode_noalloc, out, "pa_poly_decode_noalloc", ctypes.byref(D))
         return out
     ws_bytes = lib.pa_poly_decode_workspace(ctypes.byref(D))
     ws = torch.empty(max(ws_bytes, 1), dtype=torch.uint8, device=out.device)
     D.workspace, D.workspace_bytes = ws.data_ptr(), ws_bytes
-    with _device(out):
-        _lib.check(lib.pa_poly_decode(ctypes.byref(D), _stream(out)), "pa_poly_decode")
+    _call(lib.pa_poly_decode, out, "pa_poly_decode", ctypes.byref(D))
     return out
 
 
@@ -1425,5 +1466,4 @@ def decode_prologue(items, *, eps: float, angles: Optional[Tensor], n_dev: Tenso
             it.out = _view(out)
         if cache is not None:
             it.cache = _view(cache)
-    with _device(src0):
-        _lib.check(lib.pa_decode_prologue(ctypes.byref(P), _stream(src0)), "pa_decode_prologue")
+    _call(lib.pa_decode_prologue, src0, "pa_decode_prologue", ctypes.byref(P))
