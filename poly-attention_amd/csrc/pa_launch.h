@@ -44,6 +44,9 @@ void launch_mfma_fwd(const PassDev& P, int dtype, hipStream_t s);
 // are pass 1's queries / output / lse; the caller checks the views)
 bool mfma_order2_short_applies(const PassDev& P1, const PassDev& P2, int dtype);
 void launch_order2_short(const PassDev& P1, const PassDev& P2, int dtype, hipStream_t s);
+// the f16 instantiations, in a source file of their own
+void launch_mfma_fwd_f16(const PassDev& P, hipStream_t s);
+void launch_order2_short_f16(const PassDev& P1, const PassDev& P2, hipStream_t s);
 bool mfma_bwd_supported(const GradDev& G, int dtype);
 bool mfma_bwd_fuses_pre(const GradDev& G);
 // the direct-to-LDS forward / both direct-to-LDS backward kernels take this 16-bit pass (whose value
