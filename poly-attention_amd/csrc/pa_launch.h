@@ -56,6 +56,7 @@ bool mfma_bwd_dma_applies(const GradDev& G);
 // out [batch, hv, nk, dim] = v * vmul rounded to the pass dtype (16-bit)
 void launch_value_mul(const PassDev& P, void* out, int hv, int dtype, hipStream_t s);
 void launch_mfma_bwd(const GradDev& G, int dtype, hipStream_t s);
+void launch_mfma_bwd_f16(const GradDev& G, hipStream_t s);  // in a source file of its own
 
 // decode
 struct DecodeDev;
