@@ -268,7 +268,7 @@ typedef struct pa_prologue {
  * gradient summed over all rows in fp32, deterministically (workspace:
  * pa_rmsnorm_bwd_workspace bytes); with angles, dy is the gradient of the rotated output and
  * is first rotated back (rounded to the dtype, as the gradient of t).  dim must be a multiple
- * of 8 (4 for fp32) and <= 512; views need 16-byte aligned rows. */
+ * of 8 (4 for fp32) and <= 512 (256 for fp32); views need 16-byte aligned rows. */
 typedef struct pa_rmsnorm {
     int32_t     batch, heads, n, dim;
     float       eps;

@@ -362,7 +362,7 @@ static int rms_setup(const pa_rmsnorm* p, RmsDev& R, bool bwd) {
     const int T = p->x.dtype;
     if (T != PA_F32 && T != PA_F16 && T != PA_BF16) return PA_EINVAL;
     const int es = T == PA_F32 ? 4 : 2, E = 16 / es;
-    if (p->dim % E != 0 || p->dim > 512) return PA_EUNSUPPORTED;
+    if (p->dim % E != 0 || p->dim > 64 * E) return PA_EUNSUPPORTED;  // a row is within one wave
     auto view_ok = [&](const pa_view& v) {
         if (!v.ptr || v.dtype != T || v.heads != p->heads) return false;
         return (uintptr_t)v.ptr % 16 == 0 && v.sb % E == 0 && v.sh % E == 0 && v.sn % E == 0;

@@ -597,7 +597,7 @@ def rms_layout_supported(x: Tensor, weight: Optional[Tensor],
         return False
     e = 4 if x.dtype == torch.float32 else 8
     d = x.shape[-1]
-    if d % e or d > 512 or x.stride(-1) != 1 or x.numel() == 0:
+    if d % e or d > 64 * e or x.stride(-1) != 1 or x.numel() == 0:
         return False
     if any(st % e for st in x.stride()[:3]):
         return False
