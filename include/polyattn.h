@@ -400,6 +400,12 @@ int    pa_rmsnorm_fwd(const pa_rmsnorm* r, void* stream);
  * needed (inference, prefill). */
 #define PA_RMS_MAX_ITEMS 4
 int    pa_rmsnorm_fwd_many(const pa_rmsnorm* items, int count, void* stream);
+/* The norms of a layer in training: up to PA_RMS_MAX_ITEMS forwards, or with `backward` backwards
+ * (one launch, and one for the weight gradients), of one dtype and dim, all with rotary angles or
+ * all without.  In the backward each dweight receives its weight's dtype (rounded once from the
+ * fp32 sum), and items[0].workspace holds pa_rmsnorm_many_workspace bytes for all of them. */
+int    pa_rmsnorm_many(const pa_rmsnorm* items, int count, int backward, void* stream);
+size_t pa_rmsnorm_many_workspace(const pa_rmsnorm* items, int count);
 size_t pa_rmsnorm_bwd_workspace(const pa_rmsnorm* r);
 int    pa_rmsnorm_bwd(const pa_rmsnorm* r, void* stream);
 int    pa_linear_small(const pa_linear* l, void* stream);

@@ -645,6 +645,16 @@ int pa_rmsnorm_fwd_many(const pa_rmsnorm* items, int count, void* stream) {
     return finish_launch();
 }
 
+int pa_rmsnorm_many(const pa_rmsnorm* items, int count, int backward, void* stream) {
+    const int st = launch_rms_many(items, count, backward != 0, static_cast<hipStream_t>(stream));
+    if (st != PA_OK) return st;
+    return finish_launch();
+}
+
+size_t pa_rmsnorm_many_workspace(const pa_rmsnorm* items, int count) {
+    return rms_many_workspace(items, count);
+}
+
 size_t pa_rmsnorm_bwd_workspace(const pa_rmsnorm* r) {
     if (!r) return 0;
     return rms_bwd_workspace(r);

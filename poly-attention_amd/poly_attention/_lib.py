@@ -61,6 +61,8 @@ EXPORTED_SYMBOLS = (
     "pa_decode_prologue",
     "pa_rmsnorm_fwd",
     "pa_rmsnorm_fwd_many",
+    "pa_rmsnorm_many",
+    "pa_rmsnorm_many_workspace",
     "pa_rmsnorm_bwd_workspace",
     "pa_rmsnorm_bwd",
     "pa_linear_small",
@@ -330,6 +332,10 @@ def _configure(lib) -> None:
     lib.pa_rmsnorm_fwd.argtypes = [ctypes.POINTER(PaRmsNorm), c_void_p]
     lib.pa_rmsnorm_fwd_many.restype = c_int
     lib.pa_rmsnorm_fwd_many.argtypes = [ctypes.POINTER(PaRmsNorm), c_int, c_void_p]
+    lib.pa_rmsnorm_many.restype = c_int
+    lib.pa_rmsnorm_many.argtypes = [ctypes.POINTER(PaRmsNorm), c_int, c_int, c_void_p]
+    lib.pa_rmsnorm_many_workspace.restype = c_size_t
+    lib.pa_rmsnorm_many_workspace.argtypes = [ctypes.POINTER(PaRmsNorm), c_int]
     lib.pa_rmsnorm_bwd_workspace.restype = c_size_t
     lib.pa_rmsnorm_bwd_workspace.argtypes = [ctypes.POINTER(PaRmsNorm)]
     lib.pa_rmsnorm_bwd.restype = c_int

@@ -731,6 +731,85 @@ def rms_norm_many(xs: Sequence[Tensor], weights: Sequence[Optional[Tensor]],
     return ys
 
 
+def _rms_layer_fwd(xs, weights, eps, angles, keep_rstd):
+    """The norms of a layer in one launch: (ys, rstds or None)."""
+    lib = _lib.load()
+    xs = [_aligned16(x) for x in xs]
+    ys = [_empty_heads(x.shape, x) for x in xs]
+    rstds = ([torch.empty(x.shape[:3], dtype=torch.float32, device=x.device) for x in xs]
+             if keep_rstd else [None] * len(xs))
+    items = (PaRmsNorm * len(xs))(*(_rms_struct(x, w, e, angles, y=y, rstd=r)
+                                    for x, w, e, y, r in zip(xs, weights, eps, ys, rstds)))
+    _call(lib.pa_rmsnorm_many, xs[0], "pa_rmsnorm_many", items, len(xs), 0)
+    return ys, rstds
+
+
+class _RmsLayerNode(torch.autograd.Function):
+    """The q/k norms of a layer, with the rotary angles, as one autograd node: one launch forward,
+    one (and one for the weight gradients) backward."""
+
+    @staticmethod
+    def forward(ctx, angles, eps, *inputs):
+        k = len(inputs) // 2
+        xs, weights = inputs[:k], inputs[k:]
+        ys, rstds = _rms_layer_fwd(xs, weights, eps, angles, True)
+        ctx.save_for_backward(*inputs, *rstds, angles)
+        ctx.eps = eps
+        ctx.slots = [slot_ref(x) for x in xs]
+        ctx.set_materialize_grads(False)
+        return tuple(ys)
+
+    @staticmethod
+    @torch.autograd.function.once_differentiable
+    def backward(ctx, *dys):
+        *saved, angles = ctx.saved_tensors
+        k = len(saved) // 3
+        xs, weights, rstds = saved[:k], saved[k:2 * k], saved[2 * k:]
+        if any(dy is None for dy in dys):  # an unused norm: the others one by one
+            res = [(None, None) if dy is None else
+                   _rms_bwd_raw(dy, x, w, r, e, angles, claim_slot(s, x))
+                   for dy, x, w, r, e, s in zip(dys, xs, weights, rstds, ctx.eps, ctx.slots)]
+            return (None, None, *[r[0] for r in res], *[r[1] for r in res])
+        lib = _lib.load()
+        align = 4 if xs[0].dtype == torch.float32 else 8
+        grads, dxs, dws, keep = [], [], [], []
+        for dy, x, w, r, e, s in zip(dys, xs, weights, rstds, ctx.eps, ctx.slots):
+            if dy.stride(-1) != 1 or any(st % align for st in dy.stride()[:3]):
+                dy = dy.contiguous()
+            dy, xa = _aligned16(dy), _aligned16(x)
+            dx = claim_slot(s, x)
+            if dx is None or not rms_layout_supported(dx, w) or dx.data_ptr() % 16:
+                dx = _empty_heads(x.shape, x)
+            dw = torch.empty_like(w)
+            grads.append(_rms_struct(xa, w, e, angles, rstd=r, dy=dy, dx=dx, dweight=dw))
+            dxs.append(dx)
+            dws.append(dw)
+            keep += [dy, xa]
+        items = (PaRmsNorm * k)(*grads)
+        ws_bytes = lib.pa_rmsnorm_many_workspace(items, k)
+        ws = torch.empty(max(ws_bytes, 1), dtype=torch.uint8, device=xs[0].device)
+        items[0].workspace, items[0].workspace_bytes = ws.data_ptr(), ws_bytes
+        _call(lib.pa_rmsnorm_many, xs[0], "pa_rmsnorm_many", items, k, 1)
+        return (None, None, *dxs, *dws)
+
+
+def rms_norm_layer(xs: Sequence[Tensor], weights: Sequence[Tensor], eps: Sequence[Optional[float]],
+                   angles: Optional[Tensor] = None) -> Optional[list[Tensor]]:
+    """rms_norm of up to PA_RMS_MAX_ITEMS tensors of one dtype and head dim, with the same angles, in
+    one launch each way; None where that does not apply (the caller checks rms_supported)."""
+    if not 1 <= len(xs) <= _lib.PA_RMS_MAX_ITEMS or not _plain_eager(*xs, *weights, angles):
+        return None
+    x0 = xs[0]
+    if any(x.dtype != x0.dtype or x.shape[-1] != x0.shape[-1] or x.device != x0.device for x in xs):
+        return None
+    if any(w is None for w in weights):
+        return None
+    eps = tuple(torch.finfo(torch.float32).eps if e is None else float(e) for e in eps)
+    if _needs_op(*xs, *weights):
+        return list(_RmsLayerNode.apply(angles, eps, *xs, *weights))
+    return _rms_layer_fwd(xs, weights, eps, angles, False)[0]
+
+
 # ---------------------------------------------------------------------------------------
 # projections of a single-token decode step
 

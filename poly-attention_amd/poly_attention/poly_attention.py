@@ -50,9 +50,11 @@ def _q_norms(module, norms, qs, rotary_pos_emb=None):
     """The per-head q/k RMSNorms (poly_attention.py:271, n_poly_attention.py:188), then the
     external rotary when given (:275-276, :190-191): on the fused GPU path through pa_rmsnorm
     (forward and backward, the rotation inside the same kernel), else torch.nn.RMSNorm and
-    apply_rotary_emb.  Without gradients and rotary the norms of a layer go out in one launch
-    (pa_rmsnorm_fwd_many)."""
+    apply_rotary_emb.  The norms of a layer go out in one launch (pa_rmsnorm_fwd_many, with
+    gradients or rotary pa_rmsnorm_many)."""
     many = _q_norms_one_launch(module, norms, qs, rotary_pos_emb)
+    if many is None:
+        many = _q_norms_layer(module, norms, qs, rotary_pos_emb)
     if many is not None:
         return many
     out = []
@@ -99,6 +101,19 @@ def _module_angles(module, qs, rotary_pos_emb, cache):
     if not all(_ops.rms_supported(q, n.weight, angles) for n, q in zip(module.q_norms, qs)):
         return None
     return angles
+
+
+def _q_norms_layer(module, norms, qs, rotary_pos_emb):
+    """The norms of ``qs`` with the rotary as one autograd node (_ops.rms_norm_layer) when every one
+    is an RMSNorm over the head dim of a tensor pa_rmsnorm takes with these angles.  Else None."""
+    from . import _ops
+
+    if not all(isinstance(n, RMSNorm) and n.weight is not None and module._use_fused(q)
+               and tuple(n.normalized_shape) == (q.shape[-1],)
+               and _ops.rms_supported(q, n.weight, rotary_pos_emb) for n, q in zip(norms, qs)):
+        return None
+    many = _ops.rms_norm_layer(qs, [n.weight for n in norms], [n.eps for n in norms], rotary_pos_emb)
+    return None if many is None else tuple(many)
 
 
 def _q_norms_one_launch(module, norms, qs, rotary_pos_emb):
