@@ -409,6 +409,9 @@ size_t pa_rmsnorm_many_workspace(const pa_rmsnorm* items, int count);
 size_t pa_rmsnorm_bwd_workspace(const pa_rmsnorm* r);
 int    pa_rmsnorm_bwd(const pa_rmsnorm* r, void* stream);
 int    pa_linear_small(const pa_linear* l, void* stream);
+/* The same without input steps, activations and residuals, for 16-bit types, up to 64 rows and
+ * any in_features that is a multiple of 8 (the projections of a step over a larger batch). */
+int    pa_linear_rows(const pa_linear* l, void* stream);
 
 #ifdef __cplusplus
 }

@@ -667,6 +667,13 @@ int pa_rmsnorm_bwd(const pa_rmsnorm* r, void* stream) {
     return finish_launch();
 }
 
+int pa_linear_rows(const pa_linear* l, void* stream) {
+    if (!l) return PA_EINVAL;
+    const int st = launch_linear_rows(l, static_cast<hipStream_t>(stream));
+    if (st != PA_OK) return st;
+    return finish_launch();
+}
+
 int pa_linear_small(const pa_linear* l, void* stream) {
     if (!l) return PA_EINVAL;
     const int st = launch_linear_small(l, static_cast<hipStream_t>(stream));

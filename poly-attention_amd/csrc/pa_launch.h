@@ -73,5 +73,6 @@ int launch_rms_many(const pa_rmsnorm* items, int count, bool bwd, hipStream_t s)
 size_t rms_bwd_workspace(const pa_rmsnorm* p);
 int launch_rms_bwd(const pa_rmsnorm* p, hipStream_t s);
 int launch_linear_small(const pa_linear* l, hipStream_t s);
+int launch_linear_rows(const pa_linear* l, hipStream_t s);
 
 }  // namespace pa

@@ -16,6 +16,7 @@
 
 #include "pa_common.h"
 #include "pa_launch.h"
+#include "pa_mfma.h"
 
 namespace pa {
 
@@ -364,6 +365,157 @@ int launch_linear_small(const pa_linear* l, hipStream_t s) {
     if (T == PA_F32) launch_lin_t<float>(L, blocks, lds, s);
     else if (T == PA_F16) launch_lin_t<f16>(L, blocks, lds, s);
     else launch_lin_t<bf16>(L, blocks, lds, s);
+    return PA_OK;
+}
+
+// ---------------------------------------------------------------------------------------
+// A group of projections of up to 64 rows, or of fewer whose x does not fit the staging above: still
+// a pass over the weights, on the matrix cores.  A workgroup owns 16 output features, or 32 where
+// 16 give more workgroups than CUs (half the reads of x, which come through the L2 and are what
+// bounds it: 29.0 -> 23.1 us), and its eight waves share the input features, 64 a step in turn, two
+// to four steps in flight; a load of a wave takes 64 contiguous bytes of each of 16 rows.  The
+// waves' sums meet in LDS in a fixed order; fp32 sums, the bias in fp32, one rounding.
+// 32 rows of 4096 by 4096 + 1024 + 2048 features: concatenated weights and one library GEMM 57.5 us,
+// three GEMMs 36.9, this 23.1 (floor 11.4); 1024 by 1024 + 2048 + 2048: 19.6, 24.2, 8.1.  64 rows:
+// 58.8, 43.3, 31.0 and 20.0, 25.3, 10.4.  A single product stays with the library (4096 by 4096:
+// 12.4 us against 16.4).
+constexpr int kRowsWaves = 8;
+constexpr int kRowsMax = 64;
+constexpr int kRowsStep = 64;  // input features of a wave per step
+
+template <typename T, int MT, int NT>
+__global__ __launch_bounds__(kRowsWaves * 64) void k_linear_rows(LinDev L) {
+    constexpr int F = 16, R = 4;       // 16x16x32: features of a tile, sums per lane and tile
+    constexpr int J = kRowsStep / 32;  // 16-byte loads, and MFMAs, per step
+    constexpr int U = MT * NT == 8 ? 2 : 4;  // steps in flight
+    constexpr int S = NT * MT * R;     // sums per lane
+    typedef typename Mma<T>::frag frag;
+    typedef float accv __attribute__((ext_vector_type(R)));
+    __shared__ float s_sum[kRowsWaves][S][64];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int fl = lane % F, kg = lane / F;
+    int oi = 0;
+#pragma unroll
+    for (int j = 1; j < PA_LINEAR_MAX_OUT; ++j)
+        if (j < L.count && (int)blockIdx.x >= L.o[j].blk0) oi = j;
+    const LinOut O = L.o[oi];
+    const int n0 = ((int)blockIdx.x - O.blk0) * F * NT;
+    const T* w[NT];
+#pragma unroll
+    for (int n = 0; n < NT; ++n) w[n] = reinterpret_cast<const T*>(O.w) + (int64_t)min(n0 + n * F + fl, O.n - 1) * O.ws;
+    const T* x[MT];
+#pragma unroll
+    for (int m = 0; m < MT; ++m)
+        x[m] = reinterpret_cast<const T*>(L.x) + (int64_t)min(m * F + fl, L.rows - 1) * L.xs;
+    accv acc[NT][MT];
+#pragma unroll
+    for (int n = 0; n < NT; ++n)
+#pragma unroll
+        for (int m = 0; m < MT; ++m)
+#pragma unroll
+            for (int r = 0; r < R; ++r) acc[n][m][r] = 0.f;
+    // rows and features past the end repeat the last one and are not written; elements past the
+    // end of k are zeros on both sides.  Workgroups of an XCD start a KiB of k apart: weight rows a
+    // power of two apart would otherwise ask the same L2 channels at the same time.
+    const int steps = (L.k + kRowsStep - 1) / kRowsStep;
+    const int turn = (int)((blockIdx.x / 8 * kRowsWaves) % steps);
+    for (int i0 = wave; i0 < steps; i0 += kRowsWaves * U) {
+        frag a[U][NT][J], b[U][MT][J];
+#pragma unroll
+        for (int u = 0; u < U; ++u)
+#pragma unroll
+            for (int j = 0; j < J; ++j) {
+                const int i = i0 + u * kRowsWaves, st = i + turn < steps ? i + turn : i + turn - steps;
+                const int k = i < steps ? st * kRowsStep + j * 32 + kg * 8 : L.k;
+                const bool in = k < L.k;
+#pragma unroll
+                for (int n = 0; n < NT; ++n)
+                    a[u][n][j] = in ? __builtin_nontemporal_load(reinterpret_cast<const frag*>(w[n] + k)) : frag{};
+#pragma unroll
+                for (int m = 0; m < MT; ++m) b[u][m][j] = in ? *reinterpret_cast<const frag*>(x[m] + k) : frag{};
+            }
+#pragma unroll
+        for (int u = 0; u < U; ++u)
+#pragma unroll
+            for (int j = 0; j < J; ++j)
+#pragma unroll
+                for (int n = 0; n < NT; ++n)
+#pragma unroll
+                    for (int m = 0; m < MT; ++m) {
+                        if constexpr (std::is_same<T, f16>::value)
+                            acc[n][m] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a[u][n][j], b[u][m][j], acc[n][m], 0, 0, 0);
+                        else
+                            acc[n][m] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[u][n][j], b[u][m][j], acc[n][m], 0, 0, 0);
+                    }
+    }
+#pragma unroll
+    for (int n = 0; n < NT; ++n)
+#pragma unroll
+        for (int m = 0; m < MT; ++m)
+#pragma unroll
+            for (int r = 0; r < R; ++r) s_sum[wave][(n * MT + m) * R + r][lane] = acc[n][m][r];
+    __syncthreads();
+    // sum r of lane l: feature 4 (l / 16) + r, row l % 16
+    for (int i = threadIdx.x; i < S * 64; i += kRowsWaves * 64) {
+        const int l = i & 63, sr = i >> 6, m = sr / R % MT;
+        const int row = m * F + l % F, f = n0 + sr / R / MT * F + 4 * (l / F) + sr % R;
+        float t = 0.f;
+#pragma unroll
+        for (int v = 0; v < kRowsWaves; ++v) t += s_sum[v][sr][l];
+        if (row >= L.rows || f >= O.n) continue;
+        if (O.bias) t += to_f(reinterpret_cast<const T*>(O.bias)[f]);
+        reinterpret_cast<T*>(O.y)[(int64_t)row * O.ys + f] = (T)t;
+    }
+}
+
+template <typename T, int NT>
+static void launch_rows_t(const LinDev& L, int blocks, hipStream_t s) {
+    const dim3 g(blocks), b(kRowsWaves * 64);
+    if (L.rows <= 16) hipLaunchKernelGGL((k_linear_rows<T, 1, NT>), g, b, 0, s, L);
+    else if (L.rows <= 32) hipLaunchKernelGGL((k_linear_rows<T, 2, NT>), g, b, 0, s, L);
+    else hipLaunchKernelGGL((k_linear_rows<T, 4, NT>), g, b, 0, s, L);
+}
+
+int launch_linear_rows(const pa_linear* l, hipStream_t s) {
+    if (l->rows < 1 || l->in_features < 1 || l->count < 1 || l->count > PA_LINEAR_MAX_OUT || !l->x) return PA_EINVAL;
+    if (l->dtype != PA_F16 && l->dtype != PA_BF16) return PA_EUNSUPPORTED;
+    if (l->rows > kRowsMax || l->in_features % 8 != 0 || l->x_add || l->x_sum || l->norm) return PA_EUNSUPPORTED;
+    if ((uintptr_t)l->x % 16 != 0 || l->x_stride % 8 != 0) return PA_EUNSUPPORTED;
+    if (l->rows > 1 && l->x_stride < l->in_features) return PA_EINVAL;
+    LinDev L = {};
+    L.x = static_cast<const char*>(l->x);
+    L.xs = l->x_stride;
+    L.rows = l->rows;
+    L.k = l->in_features;
+    L.count = l->count;
+    int64_t total = 0;
+    for (int o = 0; o < l->count; ++o) {
+        const pa_linear_out& u = l->out[o];
+        if (!u.w || !u.y || u.out_features < 1 || u.w_stride < l->in_features) return PA_EINVAL;
+        if (l->rows > 1 && u.y_stride < u.out_features) return PA_EINVAL;
+        if (u.activation != PA_ACT_NONE || u.residual) return PA_EUNSUPPORTED;
+        if ((uintptr_t)u.w % 16 != 0 || u.w_stride % 8 != 0) return PA_EUNSUPPORTED;
+        if ((uintptr_t)u.y % 2 != 0 || (uintptr_t)u.bias % 2 != 0) return PA_EINVAL;
+        total += ((int64_t)u.out_features + 15) / 16;
+    }
+    if (total > (1 << 24)) return PA_EUNSUPPORTED;
+    const int tiles = total > 256 ? 2 : 1;
+    int blocks = 0;
+    for (int o = 0; o < l->count; ++o) {
+        const pa_linear_out& u = l->out[o];
+        LinOut& d = L.o[o];
+        d.w = static_cast<const char*>(u.w);
+        d.bias = static_cast<const char*>(u.bias);
+        d.y = static_cast<char*>(u.y);
+        d.ws = u.w_stride;
+        d.ys = u.y_stride;
+        d.n = u.out_features;
+        d.blk0 = blocks;
+        blocks += (u.out_features + 16 * tiles - 1) / (16 * tiles);
+    }
+    ProfScope ps("linear_rows", s);
+    if (l->dtype == PA_F16) tiles == 2 ? launch_rows_t<f16, 2>(L, blocks, s) : launch_rows_t<f16, 1>(L, blocks, s);
+    else tiles == 2 ? launch_rows_t<bf16, 2>(L, blocks, s) : launch_rows_t<bf16, 1>(L, blocks, s);
     return PA_OK;
 }
 

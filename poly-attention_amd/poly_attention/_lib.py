@@ -66,6 +66,7 @@ EXPORTED_SYMBOLS = (
     "pa_rmsnorm_bwd_workspace",
     "pa_rmsnorm_bwd",
     "pa_linear_small",
+    "pa_linear_rows",
 )
 
 
@@ -340,6 +341,8 @@ def _configure(lib) -> None:
     lib.pa_rmsnorm_bwd_workspace.argtypes = [ctypes.POINTER(PaRmsNorm)]
     lib.pa_rmsnorm_bwd.restype = c_int
     lib.pa_rmsnorm_bwd.argtypes = [ctypes.POINTER(PaRmsNorm), c_void_p]
+    lib.pa_linear_rows.restype = c_int
+    lib.pa_linear_rows.argtypes = [ctypes.POINTER(PaLinear), c_void_p]
     lib.pa_linear_small.restype = c_int
     lib.pa_linear_small.argtypes = [ctypes.POINTER(PaLinear), c_void_p]
 

@@ -908,6 +908,54 @@ def linear_small(x: Tensor, weight: Tensor, bias: Optional[Tensor] = None) -> Te
     return linear_small_group(x, [(weight, bias, False, None)])[0]
 
 
+LINEAR_ROWS_MAX = 64
+
+
+def linear_rows_supported(x: Tensor, weight: Tensor, bias: Optional[Tensor] = None) -> bool:
+    """Whether pa_linear_rows takes F.linear(x, weight, bias): plain inference on 16-bit CUDA tensors
+    of one dtype, at most 64 rows of x, in_features a multiple of 8."""
+    k = x.shape[-1] if x.dim() >= 1 else 0
+    if k == 0 or x.numel() > LINEAR_ROWS_MAX * k or x.numel() == 0 or k % 8:
+        return False
+    if not (x.is_cuda and weight.is_cuda) or x.dtype not in (torch.float16, torch.bfloat16):
+        return False
+    if weight.dtype != x.dtype or weight.dim() != 2 or weight.device != x.device or weight.shape[1] != k:
+        return False
+    if not _plain_eager(x, weight, bias) or _needs_op(x, weight, bias) or torch.is_autocast_enabled():
+        return False
+    if (weight.shape[0] == 0 or weight.stride(-1) != 1 or weight.stride(0) % 8 or weight.stride(0) < k
+            or weight.data_ptr() % 16):
+        return False
+    return bias is None or (bias.dtype == x.dtype and bias.dim() == 1 and bias.stride(0) == 1
+                            and bias.shape[0] == weight.shape[0] and bias.device == x.device)
+
+
+def linear_rows_group(x: Tensor, specs) -> list[Tensor]:
+    """[F.linear(x, weight, bias) for weight, bias in specs] on pa_linear_rows, up to four in one
+    launch (the caller checks linear_rows_supported for each)."""
+    lib = _lib.load()
+    k = x.shape[-1]
+    x2 = _rows2d(x, k, 8)
+    rows = x2.shape[0]
+    if rows > 1 and x2.stride(0) < k:
+        x2 = x2.contiguous()
+    outs = []
+    for first in range(0, len(specs), _lib.PA_LINEAR_MAX_OUT):
+        group = specs[first:first + _lib.PA_LINEAR_MAX_OUT]
+        lin = _lib.PaLinear()
+        lin.rows, lin.in_features, lin.dtype, lin.count = rows, k, DTYPE_CODE[x.dtype], len(group)
+        lin.x, lin.x_stride = x2.data_ptr(), x2.stride(0)
+        for o, (w, b) in zip(lin.out, group):
+            n = w.shape[0]
+            y = torch.empty(rows, n, dtype=x.dtype, device=x.device)
+            o.w, o.w_stride, o.out_features = w.data_ptr(), w.stride(0), n
+            o.bias = b.data_ptr() if b is not None else None
+            o.y, o.y_stride = y.data_ptr(), n
+            outs.append(y.view(*x.shape[:-1], n))
+        _call(lib.pa_linear_rows, x, "pa_linear_rows", ctypes.byref(lin))
+    return outs
+
+
 def _norm_fusable(norm: Optional[torch.nn.Module], x: Tensor) -> bool:
     if norm is None:
         return True
@@ -943,7 +991,8 @@ def linear(layer: torch.nn.Linear, x: Tensor, *, gelu: bool = False,
 
 def linear_many(layers, xs) -> list[Tensor]:
     """[layer(x) for layer, x in zip(layers, xs)], the projections of one input sharing
-    launches of pa_linear_small (up to four per launch) when every call qualifies."""
+    launches of pa_linear_small, or pa_linear_rows, (up to four per launch) when every call
+    qualifies."""
     x = xs[0]
     if x.is_cuda and all(xi is x for xi in xs) and all(
             linear_supported(x, layer.weight, layer.bias) for layer in layers):
@@ -952,6 +1001,11 @@ def linear_many(layers, xs) -> list[Tensor]:
             group = layers[i:i + _lib.PA_LINEAR_MAX_OUT]
             outs += linear_small_group(x, [(l.weight, l.bias, False, None) for l in group])
         return outs
+    if len(layers) > 1 and all(xi is x for xi in xs) and not (
+            torch.nn.modules.module._global_forward_hooks
+            or torch.nn.modules.module._global_forward_pre_hooks) and all(
+            _plain_linear(l) and linear_rows_supported(x, l.weight, l.bias) for l in layers):
+        return linear_rows_group(x, [(l.weight, l.bias) for l in layers])
     return [linear(layer, xi) for layer, xi in zip(layers, xs)]
 
 
@@ -1165,6 +1219,11 @@ def project_heads(layers, xs, splits):
             and not torch.nn.modules.module._global_forward_pre_hooks
             and all(_plain_linear(l) and l.bias is None for l in layers)
             and len({l.weight.dtype for l in layers}) == 1)
+    if fuse and all(linear_rows_supported(x, l.weight) for l in layers):
+        # few rows: each weight is read once, where the concatenation reads and writes them all
+        # before the GEMM reads them again (times at the kernel)
+        ys = linear_rows_group(x, [(l.weight, None) for l in layers])
+        return [list(_split_heads(y, (h,) * p, di)) for y, (p, h), di in zip(ys, splits, d)]
     if fuse:
         w = _concat_weights(layers)
         heads = tuple(h for p, h in splits for _ in range(p))
