@@ -494,6 +494,14 @@ def _plain_eager(*ts) -> bool:
 _PLAIN = (Tensor, torch.nn.Parameter)
 
 
+def _plain_grads(*ts) -> bool:
+    """_plain_eager for the gradients that reach a node: not the batches of
+    torch.autograd.grad(..., is_grads_batched=True) either, which have no memory of their own (the
+    custom ops are called once per gradient there)."""
+    return _plain_eager(*ts) and not any(
+        t is not None and torch._C._functorch.is_legacy_batchedtensor(t) for t in ts)
+
+
 class _PassNode(torch.autograd.Function):
     """polyattn::pass_fwd and its backward as one autograd node (``_plain_eager`` calls)."""
 
@@ -506,7 +514,7 @@ class _PassNode(torch.autograd.Function):
     @staticmethod
     @torch.autograd.function.once_differentiable
     def backward(ctx, dout, dlse):
-        return _pass_backward(ctx, dout, dlse, raw=True)
+        return _pass_backward(ctx, dout, dlse, raw=_plain_grads(dout, dlse))
 
 
 class _RmsNode(torch.autograd.Function):
@@ -521,7 +529,7 @@ class _RmsNode(torch.autograd.Function):
     @staticmethod
     @torch.autograd.function.once_differentiable
     def backward(ctx, dy):
-        return _rms_backward(ctx, dy, None, raw=True)
+        return _rms_backward(ctx, dy, None, raw=_plain_grads(dy))
 
 
 def _needs_op(*ts) -> bool:
@@ -765,6 +773,10 @@ class _RmsLayerNode(torch.autograd.Function):
         *saved, angles = ctx.saved_tensors
         k = len(saved) // 3
         xs, weights, rstds = saved[:k], saved[k:2 * k], saved[2 * k:]
+        if not _plain_grads(*dys):
+            res = [(None, None) if dy is None else rms_norm_bwd_op(dy, x, w, r, e, angles)
+                   for dy, x, w, r, e in zip(dys, xs, weights, rstds, ctx.eps)]
+            return (None, None, *[r[0] for r in res], *[r[1] for r in res])
         if any(dy is None for dy in dys):  # an unused norm: the others one by one
             res = [(None, None) if dy is None else
                    _rms_bwd_raw(dy, x, w, r, e, angles, claim_slot(s, x))

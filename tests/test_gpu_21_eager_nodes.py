@@ -73,3 +73,22 @@ def test_no_silent_second_derivative():
     (dq,) = torch.autograd.grad(out.float().sum(), q, create_graph=True)
     with pytest.raises(RuntimeError):
         dq.float().sum().backward()
+
+
+def test_batched_grads():
+    """is_grads_batched: each gradient of the batch as by itself, through a pass, a norm and the norms
+    of a layer."""
+    from poly_attention import _ops
+
+    q, k, v, vmul, bias = _pass_inputs()
+    w = torch.ones(64, device=dev(), dtype=torch.bfloat16, requires_grad=True)
+    out, _ = _ops.attn_pass(q, k, v, bias=bias, causal=True)
+    normed = _ops.rms_norm(q, w, None)
+    layer = _ops.rms_norm_layer([q, k], [w, w], [None, None])[1]
+    for y, xs in ((out, (q, k, v, bias)), (normed, (q, w)), (layer, (k, w))):
+        dys = randn((3, *y.shape), torch.bfloat16, 8).to(dev())
+        got = torch.autograd.grad(y, xs, dys, retain_graph=True, is_grads_batched=True, allow_unused=True)
+        for i in range(3):
+            want = torch.autograd.grad(y, xs, dys[i], retain_graph=True, allow_unused=True)
+            for a, b in zip(got, want):
+                assert torch.equal(a[i], b)
