@@ -66,29 +66,35 @@ struct DMask {
     }
 };
 
-// The score soft clamp in units of the raw scores s = q.k (so that scale * log2e times the
-// result is the log2-domain logit): tanh(a s) / a with a = scale / softclamp, by the
-// polynomial s (1 + k1 s^2 + k2 s^4 + k3 s^6) where |s| <= thr.  Filled in by soft_clamp_dev.
+// The score soft clamp of raw scores s = q.k: y = tanh(a s) with a = scale / softclamp, and the
+// log2-domain logit cl2 y (cl2 = softclamp * log2e), each by the polynomial
+// s (k[0] + k[1] s^2 + k[2] s^4 + k[3] s^6) of its own where |s| <= thr.  Filled in by soft_clamp_dev.
 struct SoftClampDev {
-    float k1, k2, k3, thr, a, ia;
+    float thr, a, cl2;
+    float y[4], l[4];
 };
 
-// tanh(y) / y on |y| <= 0.35 as 1 + c1 y^2 + c2 y^4 + c3 y^6, fitted for the least maximal
-// relative error (4.1e-8; evaluated in fp32 at most 1.3e-7 off, 4.1e-8 root mean square, as a
-// correctly rounded tanhf is within 6e-8).  A scale or softclamp whose powers leave fp32's range
-// turns the polynomial off (thr < 0: the kernels then take tanhf for every score).
+// tanh(x) / x on |x| <= 0.35 as 1 + c1 x^2 + c2 x^4 + c3 x^6, fitted for the least maximal
+// relative error (4.1e-8).  Evaluated in fp32 over unit-variance scores at d = 64 and 128, clamps 2
+// to 50: the logit at most 2.0e-7 off, root mean square 3.6e-8 to 6.2e-8, where a correctly
+// rounded tanhf and two products are 2.1e-7 off, 3.8e-8 to 6.3e-8.  A scale or softclamp whose
+// powers leave fp32's range turns the polynomial off (thr < 0: tanhf for every score).
 inline SoftClampDev soft_clamp_dev(float scale, float softclamp) {
-    SoftClampDev c = {0.f, 0.f, 0.f, -1.f, 0.f, 0.f};
+    SoftClampDev c = {-1.f, 0.f, 0.f, {0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
     if (!(softclamp > 0.f)) return c;
+    constexpr double log2e = 1.4426950408889634;
     c.a = scale / softclamp;
-    c.ia = softclamp / scale;
-    const double a2 = (double)c.a * c.a;
-    const double k3 = -4.914850154e-02 * a2 * a2 * a2, thr = 0.35 / fabs((double)c.a);
-    if (!(a2 > 1e-30) || !(fabs(k3) < 1e30) || !(fabs(k3) > 1e-36)) return c;
-    c.k1 = (float)(-3.333266316e-01 * a2);
-    c.k2 = (float)(1.329982537e-01 * a2 * a2);
-    c.k3 = (float)k3;
-    c.thr = (float)thr;
+    c.cl2 = (float)(softclamp * log2e);
+    const double a = c.a, a2 = a * a;
+    const double k[4] = {a, -3.333266316e-01 * a * a2, 1.329982537e-01 * a * a2 * a2,
+                         -4.914850154e-02 * a * a2 * a2 * a2};
+    const double lo = fmin(1.0, c.cl2), hi = fmax(1.0, c.cl2);  // y's coefficients times 1, l's cl2
+    if (!(a2 > 1e-30) || !(fabs(k[3]) * hi < 1e30) || !(fabs(k[3]) * lo > 1e-36)) return c;
+    for (int i = 0; i < 4; ++i) {
+        c.y[i] = (float)k[i];
+        c.l[i] = (float)(k[i] * softclamp * log2e);
+    }
+    c.thr = (float)(0.35 / fabs(a));
     return c;
 }
 

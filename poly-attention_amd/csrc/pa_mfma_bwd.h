@@ -37,6 +37,20 @@ constexpr int kBwdThreads = 256;
 #define PA_BWD_DMA 1  // direct-to-LDS backward kernels where they apply
 #endif
 
+// Soft-clamped passes hold y = tanh in the score registers.  The logit rounds as the forward's,
+// (score + bias) first and then lse: a bias as large as -1e9 swallows the score in both, so that
+// P = 1 for a row's only key.  The clamp's slope 1 - y^2 is held to [0, 1] (an output modifier, no
+// instruction): a masked entry has y = -inf, P = 0 whatever its bias and lse, and slope 0.
+__device__ __forceinline__ float clamp_slope(float y) {
+    return __builtin_amdgcn_fmed3f(fmaf(-y, y, 1.f), 0.f, 1.f);
+}
+
+// what a score register counts in log2 units
+template <bool SOFTCLAMP>
+__device__ __forceinline__ float score_unit(const PassDev& P) {
+    return SOFTCLAMP ? P.sc.cl2 : P.scale * kLog2e;
+}
+
 // ---------------------------------------------------------------------------------------
 // dK / dV / dbias
 
@@ -183,8 +197,7 @@ __global__ __launch_bounds__(kBwdThreads, D == 64 ? 2 : 1) void k_mfma_bwd_dkv(G
         const float x = P.bias.scalar(b, h0, key);
         bias_l2 = bias_class(x) == 0 ? x * kLog2e : -INFINITY;
     }
-    const float sl2 = P.scale * kLog2e;
-    const float ca = SOFTCLAMP ? P.sc.a : 0.f;
+    const float sl2 = score_unit<SOFTCLAMP>(P);
 
     f32x16_t dk[D / 32], dv[D / 32];
 #pragma unroll
@@ -226,7 +239,7 @@ __global__ __launch_bounds__(kBwdThreads, D == 64 ? 2 : 1) void k_mfma_bwd_dkv(G
                 }
                 // P: register i holds query qbase + 8*(i/4) + 4*hh + (i%4) of the lane's key
                 float yv[16];
-                if (SOFTCLAMP) soft_clamp16(s, P.sc);
+                if (SOFTCLAMP) soft_clamp16<false>(s, P.sc);
 #pragma unroll
                 for (int g = 0; g < 4; ++g) {
                     const float4 Lv = *reinterpret_cast<const float4*>(sL + qb * 32 + 8 * g + 4 * hh);
@@ -234,8 +247,9 @@ __global__ __launch_bounds__(kBwdThreads, D == 64 ? 2 : 1) void k_mfma_bwd_dkv(G
 #pragma unroll
                     for (int r = 0; r < 4; ++r) {
                         const int i = 4 * g + r;
-                        if (SOFTCLAMP) yv[i] = s[i] * ca;  // softclamp(s*scale) / c
-                        s[i] = fast_exp2(fmaf(s[i], sl2, bias_l2 - L[r]));
+                        if (SOFTCLAMP) yv[i] = s[i];  // tanh: softclamp(s*scale) / c
+                        s[i] = fast_exp2(SOFTCLAMP ? fmaf(s[i], sl2, bias_l2) - L[r]
+                                                   : fmaf(s[i], sl2, bias_l2 - L[r]));
                     }
                 }
                 if (CAUSAL && qbase < kw0 + 31) {  // queries before the lane's key: P = 0
@@ -254,7 +268,7 @@ __global__ __launch_bounds__(kBwdThreads, D == 64 ? 2 : 1) void k_mfma_bwd_dkv(G
                         const int i = 4 * g + r;
                         float dsv = s[i] * (dp[i] - Dd[r]);
                         dbias += dsv;
-                        if (SOFTCLAMP) dsv *= (1.f - yv[i] * yv[i]);
+                        if (SOFTCLAMP) dsv *= clamp_slope(yv[i]);
                         dp[i] = dsv;
                     }
                 }
@@ -419,11 +433,7 @@ __global__ __launch_bounds__(kBwdThreads * NG, D == 64 ? 2 : 1) void k_mfma_bwd_
         vf[c] = opaque(vf[c]);
     }
     bias_l2 = opaque(bias_l2);
-    const float sl2 = P.scale * kLog2e;
-    const float ca = SOFTCLAMP ? P.sc.a : 0.f;
-    // the score of a masked entry: its probability is 0 and, with softclamp, its factor
-    // 1 - (ca s)^2 finite
-    const float masked_s = SOFTCLAMP ? -1e9f / sl2 : -INFINITY;
+    const float sl2 = score_unit<SOFTCLAMP>(P);
     const float lmul = SOFTCLAMP ? kLog2e : -1.f / P.scale;  // lse -> seed / log2 value
     const bool need_dbias = G.dbias.ok();
 
@@ -616,7 +626,7 @@ __global__ __launch_bounds__(kBwdThreads * NG, D == 64 ? 2 : 1) void k_mfma_bwd_
 #pragma unroll
                 for (int i = 0; i < 16; ++i) {
                     const int o = 8 * (i / 4) + (i % 4);
-                    if (o < lo || o >= hi) s[i] = masked_s;
+                    if (o < lo || o >= hi) s[i] = -INFINITY;
                 }
             }
         };
@@ -632,8 +642,8 @@ __global__ __launch_bounds__(kBwdThreads * NG, D == 64 ? 2 : 1) void k_mfma_bwd_
 #pragma unroll
                     for (int r = 0; r < 4; ++r) {
                         const int i = 4 * g + r;
-                        yv[i] = s[i] * ca;
-                        s[i] = fast_exp2(fmaf(s[i], sl2, bias_l2 - L[r]));
+                        yv[i] = s[i];
+                        s[i] = fast_exp2(fmaf(s[i], sl2, bias_l2) - L[r]);
                     }
                 }
             } else {
@@ -653,7 +663,7 @@ __global__ __launch_bounds__(kBwdThreads * NG, D == 64 ? 2 : 1) void k_mfma_bwd_
             }
             if (SOFTCLAMP)
 #pragma unroll
-                for (int i = 0; i < 16; ++i) dp[i] *= (1.f - yv[i] * yv[i]);
+                for (int i = 0; i < 16; ++i) dp[i] *= clamp_slope(yv[i]);
 #pragma unroll
             for (int t2 = 0; t2 < 2; ++t2) {
                 pf[t2] = acc_to_frag<T>(s, t2);
@@ -675,11 +685,11 @@ __global__ __launch_bounds__(kBwdThreads * NG, D == 64 ? 2 : 1) void k_mfma_bwd_
         if (!SOFTCLAMP) mask(0, s0);
         scores(1, s1, dp1);
         if (SOFTCLAMP) {
-            soft_clamp16(s0, P.sc);
+            soft_clamp16<false>(s0, P.sc);
             mask(0, s0);
         }
         grads(0, s0, dp0, pf0, df0);
-        if (SOFTCLAMP) soft_clamp16(s1, P.sc);
+        if (SOFTCLAMP) soft_clamp16<false>(s1, P.sc);
         mask(1, s1);
         accumulate(0, pf0, df0);
         grads(1, s1, dp1, pf1, df1);
@@ -928,8 +938,7 @@ __global__ __launch_bounds__(kBwdThreads, D == 64 ? 2 : 1) void k_mfma_bwd_dq(Gr
     const int64_t row = ((int64_t)b * P.heads + h) * G.rsn + (q_ok ? qi : 0);
     const float lse_l2 = q_ok ? G.ws_lse[row] * kLog2e : INFINITY;
     const float dpi = q_ok ? G.ws_D[row] : 0.f;
-    const float sl2 = P.scale * kLog2e;
-    const float ca = SOFTCLAMP ? P.sc.a : 0.f;
+    const float sl2 = score_unit<SOFTCLAMP>(P);
 
     f32x16_t dq[D / 32];
 #pragma unroll
@@ -961,7 +970,7 @@ __global__ __launch_bounds__(kBwdThreads, D == 64 ? 2 : 1) void k_mfma_bwd_dq(Gr
                 }
                 // P^T: register i holds key j0 + kb*32 + 8*(i/4) + 4*hh + (i%4) of the lane's query
                 float yv[16];
-                if (SOFTCLAMP) soft_clamp16(s, P.sc);
+                if (SOFTCLAMP) soft_clamp16<false>(s, P.sc);
 #pragma unroll
                 for (int g = 0; g < 4; ++g) {
                     const float4 bb = *reinterpret_cast<const float4*>(sB + kb * 32 + 8 * g + 4 * hh);
@@ -969,8 +978,9 @@ __global__ __launch_bounds__(kBwdThreads, D == 64 ? 2 : 1) void k_mfma_bwd_dq(Gr
 #pragma unroll
                     for (int r = 0; r < 4; ++r) {
                         const int i = 4 * g + r;
-                        if (SOFTCLAMP) yv[i] = s[i] * ca;
-                        s[i] = fast_exp2(fmaf(s[i], sl2, bv[r] - lse_l2));
+                        if (SOFTCLAMP) yv[i] = s[i];
+                        s[i] = fast_exp2(SOFTCLAMP ? fmaf(s[i], sl2, bv[r]) - lse_l2
+                                                   : fmaf(s[i], sl2, bv[r] - lse_l2));
                     }
                 }
                 if (diag) {  // keys after the lane's query: P = 0
@@ -982,7 +992,7 @@ __global__ __launch_bounds__(kBwdThreads, D == 64 ? 2 : 1) void k_mfma_bwd_dq(Gr
 #pragma unroll
                 for (int i = 0; i < 16; ++i) {
                     float dsv = s[i] * (dp[i] - dpi);
-                    if (SOFTCLAMP) dsv *= (1.f - yv[i] * yv[i]);
+                    if (SOFTCLAMP) dsv *= clamp_slope(yv[i]);
                     s[i] = dsv;
                 }
 #pragma unroll
@@ -1127,11 +1137,7 @@ __global__ __launch_bounds__(kBwdThreads * NG, NG == 1 && !SOFTCLAMP ? 3 : 2) vo
     }
     lse_l2 = opaque(lse_l2);
     dpi = opaque(dpi);
-    const float sl2 = P.scale * kLog2e;
-    const float ca = SOFTCLAMP ? P.sc.a : 0.f;
-    // the score of a masked entry: its probability is 0 and, with softclamp, its factor
-    // 1 - (ca s)^2 finite
-    const float masked_s = SOFTCLAMP ? -1e9f / sl2 : -INFINITY;
+    const float sl2 = score_unit<SOFTCLAMP>(P);
 
     f32x16_t dq[D / 32];
 #pragma unroll
@@ -1275,7 +1281,7 @@ __global__ __launch_bounds__(kBwdThreads * NG, NG == 1 && !SOFTCLAMP ? 3 : 2) vo
                 lim -= 4 * hh;
 #pragma unroll
                 for (int i = 0; i < 16; ++i)
-                    if (8 * (i / 4) + (i % 4) > lim) s[i] = masked_s;
+                    if (8 * (i / 4) + (i % 4) > lim) s[i] = -INFINITY;
             }
         };
         // dS^T = P^T (dP^T - D), packed as B operands
@@ -1295,8 +1301,8 @@ __global__ __launch_bounds__(kBwdThreads * NG, NG == 1 && !SOFTCLAMP ? 3 : 2) vo
 #pragma unroll
                     for (int r = 0; r < 4; ++r) {
                         const int i = 4 * g + r;
-                        yv[i] = s[i] * ca;
-                        s[i] = fast_exp2(fmaf(s[i], sl2, bv[r] - lse_l2));
+                        yv[i] = s[i];
+                        s[i] = fast_exp2(fmaf(s[i], sl2, bv[r]) - lse_l2);
                     }
                 }
             } else {
@@ -1306,7 +1312,7 @@ __global__ __launch_bounds__(kBwdThreads * NG, NG == 1 && !SOFTCLAMP ? 3 : 2) vo
 #pragma unroll
             for (int i = 0; i < 16; ++i) {
                 float dsv = s[i] * (dp[i] - dpi);
-                if (SOFTCLAMP) dsv *= (1.f - yv[i] * yv[i]);
+                if (SOFTCLAMP) dsv *= clamp_slope(yv[i]);
                 s[i] = dsv;
             }
 #pragma unroll
@@ -1422,11 +1428,11 @@ __global__ __launch_bounds__(kBwdThreads * NG, NG == 1 && !SOFTCLAMP ? 3 : 2) vo
         if (!SOFTCLAMP) mask(0, s0);
         scores(1, s1, dp1);
         if (SOFTCLAMP) {
-            soft_clamp16(s0, P.sc);
+            soft_clamp16<false>(s0, P.sc);
             mask(0, s0);
         }
         grads(0, s0, dp0, df0);
-        if (SOFTCLAMP) soft_clamp16(s1, P.sc);
+        if (SOFTCLAMP) soft_clamp16<false>(s1, P.sc);
         mask(1, s1);
         accumulate(0, df0);
         grads(1, s1, dp1, df1);

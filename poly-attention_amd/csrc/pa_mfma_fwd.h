@@ -243,7 +243,7 @@ struct FwdWave {
     using M = Mma<T>;
     typedef typename M::frag frag;
     static constexpr int BN = TL::BN;
-    static constexpr bool PLAIN = !BIAS_IN_LOGITS;  // max taken on raw (soft-clamped) scores
+    static constexpr bool PLAIN = !BIAS_IN_LOGITS;  // max taken on raw scores (soft-clamped: logits)
 
     frag qf[D / 16];
     f32x16_t o[D / 32];
@@ -251,11 +251,16 @@ struct FwdWave {
     int kcol, hh, q0, qi, nk;
     float sl2;
 
-    // softclamp of the raw scores, before any masking (clamp-free kernels: nothing)
+    // what a score counts in log2 units: soft-clamped ones are logits already
+    static __device__ __forceinline__ float unit(const PassDev& P) {
+        return SOFTCLAMP ? 1.f : P.scale * kLog2e;
+    }
+
+    // raw scores -> soft-clamped logits, before any masking (clamp-free kernels: nothing)
     __device__ __forceinline__ void clamp(f32x16_t (&s)[KB], const PassDev& P) const {
         if constexpr (SOFTCLAMP)
 #pragma unroll
-            for (int kb = 0; kb < KB; ++kb) soft_clamp16(s[kb], P.sc);
+            for (int kb = 0; kb < KB; ++kb) soft_clamp16<true>(s[kb], P.sc);
     }
 
     // S^T block kb of a key tile: s[kb] = K[kb*32 + row, :] . Q^T
@@ -300,7 +305,7 @@ struct FwdWave {
         }
     }
 
-    // (soft-clamped) scores -> log2-domain logits in place (bias path); returns the max over the
+    // scores (soft-clamped: logits) -> log2-domain logits in place (bias path); returns the max over the
     // query's logits of this tile (PLAIN: of the raw scores, times scale*log2e)
     __device__ __forceinline__ float logits(f32x16_t (&s)[KB], const float* sB) const {
         // four independent max chains (short dependency chains), combined at the end
@@ -443,7 +448,7 @@ __global__ __launch_bounds__(kFwdThreads, D == 64 ? 2 : 1) void k_mfma_fwd(PassD
     wv.q0 = qb * kFwdBM + w * 32;
     wv.qi = wv.q0 + wv.kcol;
     wv.nk = P.nk;
-    wv.sl2 = P.scale * kLog2e;
+    wv.sl2 = W::unit(P);
     wv.m = -INFINITY;
     wv.l = 0.f;
     // Q^T operand fragments: lane (q, hh) holds Q[q][c*16 + 8*hh .. +7]
@@ -591,8 +596,8 @@ __global__ __launch_bounds__(kFwdThreads * NG, 2) void k_mfma_fwd_dma(PassDev P)
     using TL = DmaTile<D, KB>;
     constexpr int BN = TL::BN, NL = TL::NL, BM = kFwdBM * QB;
     // the key bias enters the scores as bias / scale (so that scale*log2e*(s + bias/scale) is the
-    // log2-domain logit): as the MFMA accumulator's initial value, with softclamp as the
-    // addend of its last step
+    // log2-domain logit), the MFMA accumulator's initial value; with softclamp in log2 units, as
+    // the addend of the clamp's last step
     constexpr bool FOLD = HAS_BIAS && !SOFTCLAMP;
     using W = FwdWave<T, D, KB, CAUSAL, SOFTCLAMP, HAS_BIAS, false>;
     using M = Mma<T>;
@@ -622,7 +627,7 @@ __global__ __launch_bounds__(kFwdThreads * NG, 2) void k_mfma_fwd_dma(PassDev P)
         v.q0 = wq0 + 32 * u;
         v.qi = v.q0 + kcol;
         v.nk = P.nk;
-        v.sl2 = P.scale * kLog2e;
+        v.sl2 = W::unit(P);
         v.m = -INFINITY;
         v.l = 0.f;
         const int qi = v.qi;
@@ -650,7 +655,7 @@ __global__ __launch_bounds__(kFwdThreads * NG, 2) void k_mfma_fwd_dma(PassDev P)
     const srd_t rk = make_srd(P.k.row<T>(b, h, 0), (uint32_t)(((int64_t)(P.nk - 1) * ksn + D) * 2));
     const srd_t rv = make_srd(P.v.row<T>(b, h, 0), (uint32_t)(((int64_t)(P.nk - 1) * vsn + D) * 2));
     const int bes = P.bias.dtype == PA_F32 ? 4 : 2;  // bias element size
-    const float bmul = 1.f / P.scale;
+    const float bmul = SOFTCLAMP ? kLog2e : 1.f / P.scale;
     srd_t rb = {0, 0, 0, 0};
     // (whole 16-byte chunks, the last one perhaps padding: keys past the end are dropped below)
     if (HAS_BIAS) rb = make_srd(P.bias.p + P.bias.idx(b, h, 0) * bes, (uint32_t)((P.nk * bes + 15) & ~15));
@@ -744,7 +749,7 @@ __global__ __launch_bounds__(kFwdThreads * NG, 2) void k_mfma_fwd_dma(PassDev P)
         if constexpr (SOFTCLAMP)
 #pragma unroll
             for (int kb = 0; kb < KB; ++kb)
-                soft_clamp16(s[kb], P.sc, [&](int g) __attribute__((always_inline)) {
+                soft_clamp16<true>(s[kb], P.sc, [&](int g) __attribute__((always_inline)) {
                     if (!HAS_BIAS) return make_float4(0.f, 0.f, 0.f, 0.f);
                     return *reinterpret_cast<const float4*>(&sBw[wg][kb * 32 + 8 * g + 4 * hh]);
                 });
@@ -756,7 +761,7 @@ __global__ __launch_bounds__(kFwdThreads * NG, 2) void k_mfma_fwd_dma(PassDev P)
         const T* K = sK + st * TL::ELEMS;
         const T* V = sV + st * TL::ELEMS;
         if (HAS_BIAS) {
-            // this wave's converted copy of the tile's bias: class filtered, divided by the scale
+            // this wave's converted copy of the tile's bias: class filtered, in the scores' unit
             float x;
             if (bes == 4) x = sBraw[st][lane];
             else x = (float)reinterpret_cast<const T*>(&sBraw[st][0])[lane];
@@ -1123,7 +1128,7 @@ __device__ __forceinline__ void short_block(W& wv, const PassDev& P, int q0, int
     wv.q0 = q0;
     wv.qi = q0 + wv.kcol;
     wv.nk = P.nk;
-    wv.sl2 = P.scale * kLog2e;
+    wv.sl2 = W::unit(P);
     wv.m = -INFINITY;
     wv.l = 0.f;
 #pragma unroll

@@ -55,3 +55,20 @@ def test_softclamp_short_passes(scale_softclamp, n):
     q, k, v = (randn((2, 2, n, 64), torch.bfloat16, s) for s in (8, 9, 10))
     q = (q.float() * (scale_softclamp[0] * 8.0)).to(torch.bfloat16)
     check(run_pass(q, k, v, softclamp=softclamp), torch.bfloat16, f"softclamp short {softclamp}")
+
+
+@param("dtype,d,units", ((torch.bfloat16, 64, (2, 2)), (torch.bfloat16, 64, (8, 64)),
+                         (torch.float16, 128, (1, 2))))
+@param("n", (130, 132))
+def test_softclamp_key_bias_of_minus_1e9(dtype, d, units, n):
+    """A finite key bias of -1e9 on the first key, causal: the first row's lse is -1e9 while the keys
+    after its own have biases around 0.  Their probability in the backward is 0 whatever the bias
+    and lse, and the first key's is 1, though fp32 holds no score beside 1e9.  (One such key: of
+    several, it cannot hold log n either.)  The register-staged kernels (n = 130, a bias without
+    padded rows) and the direct-to-LDS ones, these at d = 64 with both counts of wave groups (8
+    and 1024 workgroups)."""
+    q, k, v = (randn((*units, n, d), dtype, s) for s in (21, 22, 23))
+    bias = randn((*units, n), torch.float32, 24)
+    bias[..., 0] = -1e9
+    check(run_pass(q, k, v, bias=bias, causal=True, softclamp=30.0), dtype,
+          f"softclamp bias -1e9 {dtype} d={d} {units} n={n}")
