@@ -22,6 +22,7 @@ from typing import Optional, Sequence
 
 import torch
 from torch import Tensor
+from torch.utils._device import DeviceContext
 
 from . import _lib
 from ._lib import (
@@ -483,12 +484,18 @@ torch.library.register_autograd("polyattn::pass_fwd", _pass_backward, setup_cont
 
 def _plain_eager(*ts) -> bool:
     """Plain eager tensors with no transform, mode or subclass that has to see the registered custom
-    op (torch.func, vmap, dispatch modes such as fake tensors, torch.compile): the call may then
-    be an autograd node of its own, whose host time is a fraction of a custom op's."""
+    op (torch.func, vmap, dispatch modes such as fake tensors, function modes other than a
+    default device, torch.compile): the call may then be an autograd node of its own, whose host
+    time is a fraction of a custom op's."""
     return (not torch.compiler.is_compiling()
             and torch._C._functorch.peek_interpreter_stack() is None
             and torch._C._len_torch_dispatch_stack() == 0
+            and (torch._C._len_torch_function_stack() == 0 or _only_default_device())
             and all(t is None or type(t) in _PLAIN for t in ts))
+
+
+def _only_default_device() -> bool:
+    return all(type(m) is DeviceContext for m in torch.overrides._get_current_function_mode_stack())
 
 
 _PLAIN = (Tensor, torch.nn.Parameter)
