@@ -78,15 +78,18 @@ def _q_norms(module, norms, qs, rotary_pos_emb=None):
 def _module_angles(module, qs, rotary_pos_emb, cache):
     """The rotary angles of the module's own rotary embedding (poly_attention.py:302-304,
     n_poly_attention.py:224-229) for ``qs`` = (q1, ..., q_{order+1}) of one length without a cache,
-    where the q norms can apply them (pa_rmsnorm's rotation, the rounding of
-    apply_rotary_emb): every left and right query of a pass then has the positions 0 .. n - 1.
-    None where the rotation stays with the rotary module: an external rotary, a cache, other
-    lengths, learned frequencies, norms that pa_rmsnorm does not take, under torch.compile."""
+    where the q norms can apply them: every left and right query of a pass then has the positions
+    0 .. n - 1, and from fp32 frequencies pa_rmsnorm's rotation (fp32 products and sum, rounded
+    once) is apply_rotary_emb's.  None where the rotation stays with the rotary module: an
+    external rotary, a cache, other lengths, learned frequencies, frequencies of another type (a
+    layer cast whole to 16 bits: apply_rotary_emb then rounds cos, sin, each product and the sum,
+    and cached steps do too), norms that pa_rmsnorm does not take, under torch.compile."""
     rot = module.rotary_emb
     if exists(rotary_pos_emb) or exists(cache) or type(rot) is not RotaryEmbedding:
         return None
     q0 = qs[0]
-    if (torch.compiler.is_compiling() or rot.freqs.requires_grad or not module._use_fused(q0)
+    if (torch.compiler.is_compiling() or rot.freqs.requires_grad
+            or rot.freqs.dtype != torch.float32 or not module._use_fused(q0)
             or rot._forward_hooks or rot._forward_pre_hooks or torch.is_autocast_enabled("cuda")):
         return None
     from . import _ops

@@ -95,3 +95,34 @@ def test_module_rotary_prefill_cache(order):
             assert (s - t).abs().max().item() <= 1e-4
         (a, _), (b, _) = (m(x[:, 32:], cache=c, return_cache=True) for m, c in ((fused, ca), (eager, cb)))
         assert (a - b).abs().max().item() <= 1e-4
+
+
+@param("order", (2, 3))
+@param("dtype", (torch.bfloat16, torch.float16))
+@param("freqs_too", (True, False))
+def test_prefill_rotates_keys_as_the_module(order, dtype, freqs_too, monkeypatch):
+    """The rotated keys of a prefill (what the passes get) are the module's rotation of the cached,
+    unrotated ones, as a cached step rotates them: the same bits where the layer is cast whole, its
+    frequencies with it; with fp32 frequencies to one rounding (a fused product and sum)."""
+    from poly_attention import NPolyAttention, PolyAttention, _ops
+
+    kw = dict(dim=128, dim_head=64, heads=4, use_rotary_embed=True, causal=True)
+    torch.manual_seed(0)
+    layer = PolyAttention(**kw) if order == 2 else NPolyAttention(order=order, **kw)
+    freqs = layer.rotary_emb.freqs.data.clone()
+    layer = layer.to(dev()).to(dtype)
+    if not freqs_too:
+        layer.rotary_emb.freqs.data = freqs.to(dev())
+    seen = []
+    chain = _ops.poly_chain
+    monkeypatch.setattr(_ops, "poly_chain", lambda ql, qr, *a, **k: (seen.append(qr), chain(ql, qr, *a, **k))[1])
+    with torch.no_grad():
+        _, cache = layer(randn((2, 70, 128), dtype, 8).to(dev()), return_cache=True)
+        keys = cache[:2] if order == 2 else cache[0]
+        for got, raw in zip(seen[0], keys):
+            want = layer.rotary_emb.rotate_queries_or_keys(raw)
+            if freqs_too:
+                assert torch.equal(got, want)
+            else:
+                err = (got.float() - want.float()).abs()
+                assert (err <= torch.finfo(dtype).eps * want.float().abs() + 1e-6).all()
