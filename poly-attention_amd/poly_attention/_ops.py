@@ -452,15 +452,17 @@ def _pass_setup(ctx, inputs, output):
 
 
 def _pass_backward(ctx, dout, dlse, raw=False):
+    """``raw``: the call's own node, not the registered op's; plain gradients then skip the op."""
     q, k, v, vmul, bias, key_mask, query_mask, out, lse = ctx.saved_tensors
     if dout is None:
         dout = torch.zeros_like(out)
     # a q / k / v that is a piece of a head-split projection: its gradient goes straight into
-    # the projection's gradient buffer (eager only; the op is opaque to tracing)
-    outs = [claim_slot(r, t) for r, t in zip(ctx.slots, (q, k, v))]
+    # the projection's gradient buffer (plain eager only; the op is opaque to tracing)
+    plain = _plain_grads(dout, dlse)
+    outs = [claim_slot(r, t) if plain else None for r, t in zip(ctx.slots, (q, k, v))]
     if q.shape[1] != out.shape[1]:
         outs[0] = None
-    if raw or any(o is not None for o in outs):
+    if plain and (raw or any(o is not None for o in outs)):
         dq, dk, dv, dvmul, dbias = pass_bwd_raw(dout, dlse, q, k, v, vmul, bias, key_mask,
                                                 query_mask, out, lse, ctx.causal, ctx.softclamp,
                                                 ctx.scale, ctx.may_degenerate, dq_out=outs[0],
@@ -505,8 +507,11 @@ def _plain_grads(*ts) -> bool:
     """_plain_eager for the gradients that reach a node: not the batches of
     torch.autograd.grad(..., is_grads_batched=True) either, which have no memory of their own (the
     custom ops are called once per gradient there)."""
-    return _plain_eager(*ts) and not any(
-        t is not None and torch._C._functorch.is_legacy_batchedtensor(t) for t in ts)
+    return _plain_eager(*ts) and not _batched(*ts)
+
+
+def _batched(*ts) -> bool:
+    return any(t is not None and torch._C._functorch.is_legacy_batchedtensor(t) for t in ts)
 
 
 class _PassNode(torch.autograd.Function):
@@ -521,7 +526,7 @@ class _PassNode(torch.autograd.Function):
     @staticmethod
     @torch.autograd.function.once_differentiable
     def backward(ctx, dout, dlse):
-        return _pass_backward(ctx, dout, dlse, raw=_plain_grads(dout, dlse))
+        return _pass_backward(ctx, dout, dlse, raw=True)
 
 
 class _RmsNode(torch.autograd.Function):
@@ -536,7 +541,7 @@ class _RmsNode(torch.autograd.Function):
     @staticmethod
     @torch.autograd.function.once_differentiable
     def backward(ctx, dy):
-        return _rms_backward(ctx, dy, None, raw=_plain_grads(dy))
+        return _rms_backward(ctx, dy, None, raw=True)
 
 
 def _needs_op(*ts) -> bool:
@@ -700,8 +705,9 @@ def _rms_backward(ctx, dy, drstd, raw=False):
     x, weight, rstd, angles = ctx.saved_tensors
     if dy is None:
         return None, None, None, None
-    dx_out = claim_slot(ctx.slot, x)
-    if raw or dx_out is not None:  # eager: dx goes into the split projection's gradient if it can
+    plain = _plain_grads(dy)
+    dx_out = claim_slot(ctx.slot, x) if plain else None
+    if plain and (raw or dx_out is not None):  # dx into the split projection's gradient if it can
         dx, dw = _rms_bwd_raw(dy, x, weight, rstd, ctx.eps, angles, dx_out)
     else:
         dx, dw = rms_norm_bwd_op(dy, x, weight, rstd, ctx.eps, angles)
@@ -1114,13 +1120,14 @@ class _SplitHeads(torch.autograd.Function):
     def backward(ctx, *grads):
         slots = ctx.slots
         B, N, _ = slots.shape
-        if slots.buf is None:
-            # no consumer wrote in place: one concatenation (a single piece is a free view,
-            # the kernels' gradients being heads-inner)
+        if slots.buf is None or not _plain_grads(*grads):
+            # no consumer wrote in place, or a batch of gradients, which no buffer of one
+            # holds: one concatenation (a single piece is a free view, the kernels' gradients
+            # being heads-inner)
             parts = [torch.zeros(B, N, h * slots.d, dtype=slots.dtype, device=slots.device)
                      if g is None else g.transpose(1, 2).reshape(B, N, h * slots.d)
                      for g, h in zip(grads, slots.heads)]
-            slots.claimed = set()
+            slots.buf, slots.claimed = None, set()
             return (parts[0] if len(parts) == 1 else torch.cat(parts, dim=-1)), None, None, None
         for i, g in enumerate(grads):
             v = slots.view(i)
@@ -1323,6 +1330,9 @@ def order2_backward(saved, key_mask, cfg, slots, dout, dlse=None, dlse23_ext=Non
     q1, q2, q3, v3, msg, lse23, out, lse = saved
     causal, softclamp, scale = cfg
     degenerate = key_mask is not None
+    if _batched(dout, dlse, dlse23_ext, dmsg_ext):
+        raise RuntimeError("polyattn: the order-2 chain takes one gradient at a time "
+                           "(is_grads_batched is not supported)")
     if dout is None:
         dout = torch.zeros_like(out)
     # inputs that are pieces of a head-split projection get their gradients written into

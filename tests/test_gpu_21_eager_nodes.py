@@ -92,3 +92,41 @@ def test_batched_grads():
             want = torch.autograd.grad(y, xs, dys[i], retain_graph=True, allow_unused=True)
             for a, b in zip(got, want):
                 assert torch.equal(a[i], b)
+
+
+def _layer(order):
+    from poly_attention import NPolyAttention, PolyAttention
+
+    torch.manual_seed(0)
+    kw = dict(dim=128, dim_head=64, heads=2, causal=True)
+    layer = PolyAttention(**kw) if order == 2 else NPolyAttention(order=order, **kw)
+    layer = layer.to(dev()).to(torch.bfloat16)
+    x = randn((2, 40, 128), torch.bfloat16, 9).to(dev()).requires_grad_()
+    return x, layer(x), [x, *(p for p in layer.parameters() if p.requires_grad)]
+
+
+def test_batched_grads_of_a_layer():
+    """A whole order-3 layer, whose passes and norms write their gradients into the head-split
+    projection's: each gradient of the batch as by itself (to the rounding of a batched product
+    in torch), and an ordinary backward afterwards as before."""
+    x, y, xs = _layer(3)
+    dys = randn((3, *y.shape), torch.bfloat16, 10).to(dev())
+    want = [torch.autograd.grad(y, xs, dys[i], retain_graph=True) for i in range(3)]
+    got = torch.autograd.grad(y, xs, dys, retain_graph=True, is_grads_batched=True)
+    for i in range(3):
+        for a, b in zip(got, want[i]):
+            assert (a[i].float() - b.float()).norm() <= 1e-2 * b.float().norm()
+    again = torch.autograd.grad(y, xs, dys[0])
+    for a, b in zip(again, want[0]):
+        assert torch.equal(a, b)
+
+
+def test_batched_grads_of_the_order2_chain_are_refused():
+    """One node for the chain: a clear error, and the graph stays usable."""
+    x, y, xs = _layer(2)
+    dy = randn(tuple(y.shape), torch.bfloat16, 10).to(dev())
+    want = torch.autograd.grad(y, xs, dy, retain_graph=True)
+    with pytest.raises(RuntimeError, match="one gradient at a time"):
+        torch.autograd.grad(y, xs, torch.stack([dy, dy]), retain_graph=True, is_grads_batched=True)
+    for a, b in zip(torch.autograd.grad(y, xs, dy), want):
+        assert torch.equal(a, b)
