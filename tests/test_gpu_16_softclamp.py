@@ -72,3 +72,18 @@ def test_softclamp_key_bias_of_minus_1e9(dtype, d, units, n):
     bias[..., 0] = -1e9
     check(run_pass(q, k, v, bias=bias, causal=True, softclamp=30.0), dtype,
           f"softclamp bias -1e9 {dtype} d={d} {units} n={n}")
+
+
+@param("dtype", (torch.bfloat16, torch.float16))
+@param("causal", (False, True))
+@param("biased", (False, True))
+@param("softclamp", (2.0, 30.0))
+def test_softclamp_large_grids(dtype, causal, biased, softclamp):
+    """Enough heads for one group of waves per workgroup in both directions (1024 workgroups in the
+    backward, 512 of 256 queries in the forward), two query and three key tiles, the last of four
+    keys; both branches of the clamp."""
+    n = 132
+    q, k, v = (randn((8, 64, n, 64), dtype, s) for s in (25, 26, 27))
+    bias = randn((8, 64, n), torch.float32, 28) if biased else None
+    check(run_pass(q, k, v, bias=bias, causal=causal, softclamp=softclamp), dtype,
+          f"softclamp {softclamp} large grid {dtype} causal={causal} biased={biased}")

@@ -53,3 +53,44 @@ def test_value_multiplier_head_counts(hv, hm):
     ref, ref_lse = _ops.attn_pass(q, k, full.contiguous(), causal=True)
     assert_parity(out, ref.cpu(), dtype, f"head counts {hv} {hm}", tol=0.0, roundings=0)
     assert torch.equal(lse, ref_lse)
+
+
+@param("dtype,d", ((torch.bfloat16, 64), (torch.float16, 64), (torch.bfloat16, 128)))
+@param("n,padded", ((4, False), (132, False), (260, False), (63, True), (130, True), (257, True)))
+def test_value_multiplier_folded(dtype, d, n, padded):
+    """The lengths that take the folded value: a multiple of four (the bias rows of the lengths above
+    are not readable in whole 16-byte chunks, so their backward stays register-staged), or a bias
+    in padded rows, as a chain's deeper level gives it.  GQA, causal, two wave groups at d = 64."""
+    import oracle.poly_oracle as O
+    from poly_attention import _ops
+
+    q = randn((2, 4, n, d), dtype, 1)
+    k, v, vmul = (randn((2, 2, n, d), dtype, s) for s in (2, 3, 4))
+    bias = randn((2, 2, n), torch.float32, 5)
+    do, dl = randn((2, 4, n, d), dtype, 6), randn((2, 4, n), torch.float32, 7)
+    gb = torch.full((2, 2, n + (-n % 4 if padded else 0)), float("nan"), device=dev())[..., :n]
+    gb.copy_(bias)
+    assert bool(_ops._bias_flags(gb)) == padded
+    g = [t.to(dev()).requires_grad_() for t in (q, k, v, vmul)] + [gb.detach().requires_grad_()]
+    out, lse = _ops.attn_pass(*g, causal=True)
+    res = [out, *torch.autograd.grad((out, lse), g, (do.to(dev()), dl.to(dev())))]
+    refs = []
+    for dt in (torch.float32, dtype):
+        o = [t.to(dt).requires_grad_() for t in (q, k, v, vmul, bias)]
+        ro, rl = O.attn_pass(*o, causal=True)
+        refs.append([ro, *torch.autograd.grad((ro, rl), o, (do.to(ro.dtype), dl.to(rl.dtype)))])
+    for name, a, b, c in zip(("out", "dq", "dk", "dv", "dvmul", "dbias"), res, *refs):
+        assert_parity(a, b, dtype, f"vmul folded {dtype} d={d} n={n} {name}", grad=name != "out", ref_lp=c)
+
+
+@param("dtype", (torch.bfloat16, torch.float16))
+@param("causal", (False, True))
+@param("softclamp", (None, 30.0))
+def test_value_multiplier_large_grids(dtype, causal, softclamp):
+    """Enough heads for one group of waves per workgroup in the backward (1024 workgroups, past the
+    threshold of 512 causal, 128 not), where dv and dvmul are formed without a merge."""
+    n = 132
+    q, k, v, vmul = (randn((8, 64, n, 64), dtype, s) for s in (15, 16, 17, 18))
+    bias = randn((8, 64, n), torch.float32, 19)
+    check(run_pass(q, k, v, vmul=vmul, bias=bias, causal=causal, softclamp=softclamp), dtype,
+          f"vmul large grid {dtype} causal={causal} softclamp={softclamp}")
