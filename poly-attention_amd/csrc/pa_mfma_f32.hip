@@ -332,7 +332,6 @@ __global__ __launch_bounds__(64 * R * C, R * C / 4) void k_mfma_fwd_f32(PassDev 
     float m, l, big;  // big: the largest magnitude of the operands
 
     const bool sc = P.softclamp > 0.f;
-    const float sl2 = P.scale * kLog2e;
     const int kend = causal ? min(P.nk, (qb + 1) * 32 * R) : P.nk;
     const int wave_kend = causal ? min(kend, q0 + 32) : kend;
     const float* kp = P.k.row<float>(b, h, 0);
@@ -372,21 +371,20 @@ __global__ __launch_bounds__(64 * R * C, R * C / 4) void k_mfma_fwd_f32(PassDev 
                 f32x16_t s = zero16();
                 ln.template rows_mma<BIG>(K, qf, s);
                 float mx[4] = {-INFINITY, -INFINITY, -INFINITY, -INFINITY};
+#pragma unroll
+                for (int i = 0; i < 16; ++i) s[i] *= P.scale;
                 if (sc) {
                     keep_branch();
 #pragma unroll
-                    for (int i = 0; i < 16; ++i) s[i] = softclamp_f(s[i] * P.scale, P.softclamp) * kLog2e;
-                } else {
-#pragma unroll
-                    for (int i = 0; i < 16; ++i) s[i] *= sl2;
+                    for (int i = 0; i < 16; ++i) s[i] = softclamp_f(s[i], P.softclamp);
                 }
 #pragma unroll
-                for (int g = 0; g < 4; ++g) {
+                for (int g = 0; g < 4; ++g) {  // one rounding, as in the backward
                     const float4 bb = *reinterpret_cast<const float4*>(B + 8 * g + 4 * ln.hh);
-                    s[4 * g] += bb.x;
-                    s[4 * g + 1] += bb.y;
-                    s[4 * g + 2] += bb.z;
-                    s[4 * g + 3] += bb.w;
+                    s[4 * g] = fmaf(s[4 * g], kLog2e, bb.x);
+                    s[4 * g + 1] = fmaf(s[4 * g + 1], kLog2e, bb.y);
+                    s[4 * g + 2] = fmaf(s[4 * g + 2], kLog2e, bb.z);
+                    s[4 * g + 3] = fmaf(s[4 * g + 3], kLog2e, bb.w);
                 }
                 if (causal && j0 + 31 > q0) {
                     keep_branch();
