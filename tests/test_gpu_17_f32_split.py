@@ -76,3 +76,79 @@ def test_infinite_and_huge_values(d):
     ref, _ = O.attn_pass(q.double(), k.double(), v.double(), causal=True)
     rows, feats = slice(0, 32), [f for f in range(d) if f != 5]
     assert ((out[0, 0, rows, feats].cpu().double() - ref[0, 0, rows, feats]).abs() <= 1e-4).all()
+
+
+def _grads(run, q, k, v, bias, do):
+    ts = [t.requires_grad_() for t in (q, k, v, bias)]
+    out = run(*ts)
+    return [out.detach(), *torch.autograd.grad(out, ts, do)]
+
+
+@param("d", (64, 128))
+@param("causal", (False, True))
+@param("where", ("q", "k", "v", "do"))
+def test_backward_of_huge_values(d, causal, where):
+    """A finite element that bf16 cannot hold sends dQ or dK/dV (whichever has it as an operand) over
+    its tiles again, from zero accumulators, dbias and the first head and stage (GQA: two query
+    heads per key head, several stages).  Its feature is zero in the tensor it is multiplied with,
+    so every score and dP stays ordinary, and its own products are finite: every result against 64
+    bits, the element's feature by itself, at test_accuracy_against_64_bits's 2e-6."""
+    from poly_attention import _ops
+
+    n, f = 300, 9
+    q, do = (randn((1, 4, n, d), torch.float32, s) for s in (16, 17))
+    k, v = (randn((1, 2, n, d), torch.float32, s) for s in (18, 19))
+    bias = randn((1, 2, n), torch.float32, 20)
+    ts = {"q": q, "k": k, "v": v, "do": do}
+    ts[{"q": "k", "k": "q", "v": "do", "do": "v"}[where]][..., f] = 0.0
+    ts[where][0, 1, 150, f] = 3.39e38
+    got = _grads(lambda *a: _ops.attn_pass(*a[:3], bias=a[3], causal=causal)[0],
+                 *(t.to(dev()) for t in (q, k, v, bias)), do.to(dev()))
+    ref = _grads(lambda *a: O.attn_pass(*a[:3], bias=a[3], causal=causal)[0],
+                 *(t.double() for t in (q, k, v, bias)), do.double())
+    rest = [i for i in range(d) if i != f]
+    for name, a, b in zip(("out", "dq", "dk", "dv", "dbias"), got, ref):
+        a = a.cpu().double()
+        for part in ((rest, [f]) if a.dim() == 4 else (None,)):
+            x, y = (a, b) if part is None else (a[..., part], b[..., part])
+            assert torch.isfinite(x).all(), f"{name} {part}"
+            assert (x - y).norm() <= 2e-6 * y.norm(), f"{name} of a huge {where} element, {part}"
+
+
+@param("d", (64, 128))
+def test_backward_of_an_infinite_gradient(d):
+    """An infinite element of dout: its row's dP and D are infinite, so dq of the row and every dk of
+    its key head are not finite; dv of its feature is infinite, and every other dq row, dk and dv
+    is as in 64 bits."""
+    from poly_attention import _ops
+
+    n, f, i = 100, 5, 40
+    q, do = (randn((1, 4, n, d), torch.float32, s) for s in (21, 22))
+    k, v = (randn((1, 2, n, d), torch.float32, s) for s in (23, 24))
+    bias = randn((1, 2, n), torch.float32, 25)
+    do[0, 3, i, f] = float("inf")
+    got = _grads(lambda *a: _ops.attn_pass(*a[:3], bias=a[3])[0], *(t.to(dev()) for t in (q, k, v, bias)),
+                 do.to(dev()))
+    ref = _grads(lambda *a: O.attn_pass(*a[:3], bias=a[3])[0], *(t.double() for t in (q, k, v, bias)),
+                 do.double())
+    for name, a, b in zip(("out", "dq", "dk", "dv", "dbias"), got, ref):
+        a, fin = a.cpu().double(), torch.isfinite(b)
+        assert torch.equal(torch.isfinite(a), fin), name
+        if name == "dv":
+            assert torch.equal(a[~fin], b[~fin]) and (~fin).sum() == n
+        assert (a[fin] - b[fin]).norm() <= 2e-6 * b[fin].norm(), name
+
+
+@param("scale", (1e-30, 2.0 ** -100, 1e30))
+def test_accuracy_of_extreme_magnitudes(scale):
+    """The three parts hold all 24 bits down to 2^-110 (the third is then bf16's smallest number,
+    2^-133) and up to the largest; as test_accuracy_against_64_bits."""
+    from poly_attention import _ops
+
+    q, k, v, do = (randn((1, 4, 300, 64), torch.float32, s) for s in (26, 27, 28, 29))
+    v = v * scale
+    ts = [t.to(dev()).requires_grad_() for t in (q, k, v)]
+    out, _ = _ops.attn_pass(*ts, causal=True)
+    got = [out.detach(), *torch.autograd.grad(out, ts, do.to(dev()))]
+    for a, b in zip(got, _pass64(q, k, v, do)):
+        assert ((a.double().cpu() - b).norm() / b.norm()).item() < 2e-6
