@@ -116,7 +116,7 @@ PassDev to_passdev(const pa_pass* p) {
     P.dim = p->dim;
     P.scale = p->scale;
     P.softclamp = p->softclamp;
-    P.sc = soft_clamp_dev(p->scale, p->softclamp);
+    P.sc = soft_clamp_dev(p->scale, p->softclamp, /*logit=*/true);
     P.causal = p->causal;
     P.flags = p->flags;
     P.q = to_dview(p->q, p->heads);
@@ -491,6 +491,7 @@ int pa_attn_pass_bwd(const pa_pass_grad* g, void* stream) {
 
     GradDev G;
     G.f = to_passdev(p);
+    G.f.sc = soft_clamp_dev(p->scale, p->softclamp, /*logit=*/false);
     G.dout = to_dview(g->dout, H);
     G.dlse = to_dview(g->dlse, H);
     G.dq = to_dview(g->dq, H);

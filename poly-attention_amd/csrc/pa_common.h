@@ -66,12 +66,13 @@ struct DMask {
     }
 };
 
-// The score soft clamp of raw scores s = q.k: y = tanh(a s) with a = scale / softclamp, and the
-// log2-domain logit cl2 y (cl2 = softclamp * log2e), each by the polynomial
-// s (k[0] + k[1] s^2 + k[2] s^4 + k[3] s^6) of its own where |s| <= thr.  Filled in by soft_clamp_dev.
+// The score soft clamp of raw scores s = q.k, a = scale / softclamp: y = tanh(a s) in the backward, the
+// log2-domain logit cl2 y (cl2 = softclamp * log2e) in the forward, by the polynomial
+// s (k[0] + k[1] s^2 + k[2] s^4 + k[3] s^6) where |s| <= thr.  Filled in by soft_clamp_dev.
 struct SoftClampDev {
-    float thr, a, cl2;
-    float y[4], l[4];
+    float k[4];  // backward: k[0] = a
+    float thr;
+    float u;     // forward: a; backward: cl2 (from here it stays in a scalar register)
 };
 
 // tanh(x) / x on |x| <= 0.35 as 1 + c1 x^2 + c2 x^4 + c3 x^6, fitted for the least maximal
@@ -79,22 +80,20 @@ struct SoftClampDev {
 // to 50: the logit at most 2.0e-7 off, root mean square 3.6e-8 to 6.2e-8, where a correctly
 // rounded tanhf and two products are 2.1e-7 off, 3.8e-8 to 6.3e-8.  A scale or softclamp whose
 // powers leave fp32's range turns the polynomial off (thr < 0: tanhf for every score).
-inline SoftClampDev soft_clamp_dev(float scale, float softclamp) {
-    SoftClampDev c = {-1.f, 0.f, 0.f, {0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
+inline SoftClampDev soft_clamp_dev(float scale, float softclamp, bool logit) {
+    SoftClampDev c = {{0.f, 0.f, 0.f, 0.f}, -1.f, 0.f};
     if (!(softclamp > 0.f)) return c;
     constexpr double log2e = 1.4426950408889634;
-    c.a = scale / softclamp;
-    c.cl2 = (float)(softclamp * log2e);
-    const double a = c.a, a2 = a * a;
-    const double k[4] = {a, -3.333266316e-01 * a * a2, 1.329982537e-01 * a * a2 * a2,
-                         -4.914850154e-02 * a * a2 * a2 * a2};
-    const double lo = fmin(1.0, c.cl2), hi = fmax(1.0, c.cl2);  // y's coefficients times 1, l's cl2
-    if (!(a2 > 1e-30) || !(fabs(k[3]) * hi < 1e30) || !(fabs(k[3]) * lo > 1e-36)) return c;
-    for (int i = 0; i < 4; ++i) {
-        c.y[i] = (float)k[i];
-        c.l[i] = (float)(k[i] * softclamp * log2e);
-    }
-    c.thr = (float)(0.35 / fabs(a));
+    const float a = scale / softclamp;
+    c.k[0] = logit ? (float)(scale * log2e) : a;
+    c.u = logit ? a : (float)(softclamp * log2e);
+    const double a2 = (double)a * a, k0 = logit ? scale * log2e : a;
+    const double k3 = -4.914850154e-02 * a2 * a2 * a2 * k0;
+    if (!(a2 > 1e-30) || !(fabs(k3) < 1e30) || !(fabs(k3) > 1e-37)) return c;
+    c.k[1] = (float)(-3.333266316e-01 * a2 * k0);
+    c.k[2] = (float)(1.329982537e-01 * a2 * a2 * k0);
+    c.k[3] = (float)k3;
+    c.thr = (float)(0.35 / fabs((double)a));
     return c;
 }
 

@@ -84,30 +84,30 @@ __device__ __forceinline__ void keep_branch() { asm volatile("" ::: "memory"); }
 // the wave index as a scalar value, so conditions built from it compile to scalar branches
 __device__ __forceinline__ int wave_id() { return __builtin_amdgcn_readfirstlane(threadIdx.x >> 6); }
 
-// Soft clamp of one accumulator block of raw scores in place (SoftClampDev): y = tanh, or with
-// LOGIT the log2-domain logits cl2 y; register i = 4g + r also takes element r of bias(g), a float4
-// read where it is used.  tanhf costs about 30 instructions a score and used to be half the
-// kernels' time; the polynomial costs five, and a wave takes it whenever all its scores of the
-// block are in its range (|s * scale| <= 0.35 softclamp: all but outliers at the usual clamps of
+// Soft clamp of one accumulator block of raw scores in place (SoftClampDev): y = tanh (the backward),
+// or with LOGIT the log2-domain logits (the forward); register i = 4g + r also takes element r of
+// bias(g), a float4 read where it is used.  tanhf costs about 30 instructions a score and used to be
+// half the kernels' time; the polynomial costs five, and a wave takes it whenever all its scores of
+// the block are in its range (|s * scale| <= 0.35 softclamp: all but outliers at the usual clamps of
 // 30 to 50).  B = 4, H = 8, N = 1000, d = 64, causal, softclamp 50, per level: forward 93-98 ->
 // 41-52 us, dQ 62-76 -> 37-38 (with two workgroups per CU), dK/dV 65-68 -> 41-44.  Where nearly every
 // block leaves the range (softclamp 1, B = 4, H = 16, N = 2048, causal) a level's forward 252 -> 218,
 // its backward 364 -> 374: the range test, and dQ at two workgroups per CU instead of three.
 template <bool LOGIT, class Bias>
-__device__ __forceinline__ void soft_clamp16(f32x16_t& s, const SoftClampDev& c, Bias bias) {
-    const float* k = LOGIT ? c.l : c.y;
-    const float top = LOGIT ? c.cl2 : 1.f;
+__device__ __forceinline__ void soft_clamp16(f32x16_t& s, const PassDev& P, Bias bias) {
+    const SoftClampDev& c = P.sc;
     float mx = 0.f;
 #pragma unroll
     for (int i = 0; i < 16; i += 2) mx = fmaxf(fmaxf(mx, fabsf(s[i])), fabsf(s[i + 1]));
     if (__any(!(mx <= c.thr))) {
         keep_branch();
+        const float a = LOGIT ? c.u : c.k[0], top = LOGIT ? P.softclamp * kLog2e : 1.f;
 #pragma unroll
         for (int g = 0; g < 4; ++g) {
             const float4 bb = bias(g);
             const float bv[4] = {bb.x, bb.y, bb.z, bb.w};
 #pragma unroll
-            for (int r = 0; r < 4; ++r) s[4 * g + r] = fmaf(tanhf(s[4 * g + r] * c.a), top, bv[r]);
+            for (int r = 0; r < 4; ++r) s[4 * g + r] = fmaf(tanhf(s[4 * g + r] * a), top, bv[r]);
         }
     } else {
 #pragma unroll
@@ -117,14 +117,14 @@ __device__ __forceinline__ void soft_clamp16(f32x16_t& s, const SoftClampDev& c,
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
                 const float x = s[4 * g + r], z = x * x;
-                s[4 * g + r] = fmaf(x, fmaf(fmaf(fmaf(k[3], z, k[2]), z, k[1]), z, k[0]), bv[r]);
+                s[4 * g + r] = fmaf(x, fmaf(fmaf(fmaf(c.k[3], z, c.k[2]), z, c.k[1]), z, c.k[0]), bv[r]);
             }
         }
     }
 }
 template <bool LOGIT>
-__device__ __forceinline__ void soft_clamp16(f32x16_t& s, const SoftClampDev& c) {
-    soft_clamp16<LOGIT>(s, c, [](int) __attribute__((always_inline)) { return make_float4(0.f, 0.f, 0.f, 0.f); });
+__device__ __forceinline__ void soft_clamp16(f32x16_t& s, const PassDev& P) {
+    soft_clamp16<LOGIT>(s, P, [](int) __attribute__((always_inline)) { return make_float4(0.f, 0.f, 0.f, 0.f); });
 }
 
 // accumulator registers 8t .. 8t+7 (times `scale`) as a B-operand fragment

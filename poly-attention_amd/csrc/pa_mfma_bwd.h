@@ -48,7 +48,7 @@ __device__ __forceinline__ float clamp_slope(float y) {
 // what a score register counts in log2 units
 template <bool SOFTCLAMP>
 __device__ __forceinline__ float score_unit(const PassDev& P) {
-    return SOFTCLAMP ? P.sc.cl2 : P.scale * kLog2e;
+    return SOFTCLAMP ? P.sc.u : P.scale * kLog2e;
 }
 
 // ---------------------------------------------------------------------------------------
@@ -239,7 +239,7 @@ __global__ __launch_bounds__(kBwdThreads, D == 64 ? 2 : 1) void k_mfma_bwd_dkv(G
                 }
                 // P: register i holds query qbase + 8*(i/4) + 4*hh + (i%4) of the lane's key
                 float yv[16];
-                if (SOFTCLAMP) soft_clamp16<false>(s, P.sc);
+                if (SOFTCLAMP) soft_clamp16<false>(s, P);
 #pragma unroll
                 for (int g = 0; g < 4; ++g) {
                     const float4 Lv = *reinterpret_cast<const float4*>(sL + qb * 32 + 8 * g + 4 * hh);
@@ -685,11 +685,11 @@ __global__ __launch_bounds__(kBwdThreads * NG, D == 64 ? 2 : 1) void k_mfma_bwd_
         if (!SOFTCLAMP) mask(0, s0);
         scores(1, s1, dp1);
         if (SOFTCLAMP) {
-            soft_clamp16<false>(s0, P.sc);
+            soft_clamp16<false>(s0, P);
             mask(0, s0);
         }
         grads(0, s0, dp0, pf0, df0);
-        if (SOFTCLAMP) soft_clamp16<false>(s1, P.sc);
+        if (SOFTCLAMP) soft_clamp16<false>(s1, P);
         mask(1, s1);
         accumulate(0, pf0, df0);
         grads(1, s1, dp1, pf1, df1);
@@ -970,7 +970,7 @@ __global__ __launch_bounds__(kBwdThreads, D == 64 ? 2 : 1) void k_mfma_bwd_dq(Gr
                 }
                 // P^T: register i holds key j0 + kb*32 + 8*(i/4) + 4*hh + (i%4) of the lane's query
                 float yv[16];
-                if (SOFTCLAMP) soft_clamp16<false>(s, P.sc);
+                if (SOFTCLAMP) soft_clamp16<false>(s, P);
 #pragma unroll
                 for (int g = 0; g < 4; ++g) {
                     const float4 bb = *reinterpret_cast<const float4*>(sB + kb * 32 + 8 * g + 4 * hh);
@@ -1428,11 +1428,11 @@ __global__ __launch_bounds__(kBwdThreads * NG, NG == 1 && !SOFTCLAMP ? 3 : 2) vo
         if (!SOFTCLAMP) mask(0, s0);
         scores(1, s1, dp1);
         if (SOFTCLAMP) {
-            soft_clamp16<false>(s0, P.sc);
+            soft_clamp16<false>(s0, P);
             mask(0, s0);
         }
         grads(0, s0, dp0, df0);
-        if (SOFTCLAMP) soft_clamp16<false>(s1, P.sc);
+        if (SOFTCLAMP) soft_clamp16<false>(s1, P);
         mask(1, s1);
         accumulate(0, df0);
         grads(1, s1, dp1, df1);

@@ -260,7 +260,7 @@ struct FwdWave {
     __device__ __forceinline__ void clamp(f32x16_t (&s)[KB], const PassDev& P) const {
         if constexpr (SOFTCLAMP)
 #pragma unroll
-            for (int kb = 0; kb < KB; ++kb) soft_clamp16<true>(s[kb], P.sc);
+            for (int kb = 0; kb < KB; ++kb) soft_clamp16<true>(s[kb], P);
     }
 
     // S^T block kb of a key tile: s[kb] = K[kb*32 + row, :] . Q^T
@@ -749,7 +749,7 @@ __global__ __launch_bounds__(kFwdThreads * NG, 2) void k_mfma_fwd_dma(PassDev P)
         if constexpr (SOFTCLAMP)
 #pragma unroll
             for (int kb = 0; kb < KB; ++kb)
-                soft_clamp16<true>(s[kb], P.sc, [&](int g) __attribute__((always_inline)) {
+                soft_clamp16<true>(s[kb], P, [&](int g) __attribute__((always_inline)) {
                     if (!HAS_BIAS) return make_float4(0.f, 0.f, 0.f, 0.f);
                     return *reinterpret_cast<const float4*>(&sBw[wg][kb * 32 + 8 * g + 4 * hh]);
                 });

@@ -6,7 +6,7 @@ the score, is far below them)."""
 import pytest
 import torch
 
-from test_gpu_1_pass import check, randn, run_pass
+from test_gpu_1_pass import check, dev, randn, run_pass
 
 pytestmark = pytest.mark.gpu
 param = pytest.mark.parametrize
@@ -87,3 +87,22 @@ def test_softclamp_large_grids(dtype, causal, biased, softclamp):
     bias = randn((8, 64, n), torch.float32, 28) if biased else None
     check(run_pass(q, k, v, bias=bias, causal=causal, softclamp=softclamp), dtype,
           f"softclamp {softclamp} large grid {dtype} causal={causal} biased={biased}")
+
+
+@param("causal", (False, True))
+def test_softclamp_at_scale_zero(causal):
+    """A scale of 0: every visible key has the same probability, and dq and dk are 0 (a clamp held as a
+    multiple of the raw score would be 0 * inf)."""
+    from poly_attention import _ops
+
+    q, k, v, do = (randn((1, 2, 132, 64), torch.bfloat16, s).to(dev()) for s in (31, 32, 33, 34))
+    ts = [t.requires_grad_() for t in (q, k, v)]
+    out, _ = _ops.attn_pass(*ts, causal=causal, softclamp=20.0, scale=0.0)
+    dq, dk, dv = torch.autograd.grad(out, ts, do)
+    seen = torch.ones(132, 132, device=dev()).tril() if causal else torch.ones(132, 132, device=dev())
+    p = seen / seen.sum(-1, keepdim=True)
+    assert (out.float() - p @ v.detach().float()).abs().max() <= 2e-2
+    assert not dq.any() and not dk.any()
+    # P in bf16: each of up to 132 terms off by 2^-9 of itself
+    bound = 2.0 ** -8 * (p.t() @ do.float().abs()) + 2.0 ** -8 * dv.float().abs() + 1e-6
+    assert ((dv.float() - p.t() @ do.float()).abs() <= bound).all()
