@@ -35,6 +35,10 @@ bool mfma_fwd_f32_supported(const PassDev& P);
 void launch_mfma_fwd_f32(const PassDev& P, hipStream_t s);
 bool mfma_bwd_f32_supported(const GradDev& G);  // unmasked passes
 void launch_mfma_bwd_f32(const GradDev& G, hipStream_t s);
+// head dim 128 in small grids, one 32-row block of queries per workgroup (in a source file of its own)
+bool mfma_f32_block_applies(const PassDev& P, int64_t blocks);
+void launch_mfma_fwd_f32_block(const PassDev& P, int64_t blocks, hipStream_t s);
+void launch_mfma_bwd_f32_dq_block(const GradDev& G, int64_t blocks, hipStream_t s);
 bool mfma_fwd_supported(const PassDev& P, int dtype);
 // the short-pass kernel takes this pass (head dim 64, nq, nk <= 64, not causal, no value
 // multiplier or key mask, 16-bit)

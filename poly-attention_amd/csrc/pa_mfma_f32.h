@@ -1,5 +1,5 @@
-// pa_mfma_f32.h -- pieces of the fp32 attention passes on the bf16 matrix cores that their kernels share;
-// the method is described in pa_mfma_f32.hip.
+// pa_mfma_f32.h -- pieces of the fp32 attention passes on the bf16 matrix cores that their kernels share
+// (pa_mfma_f32.hip, where the method is described, and pa_mfma_f32_block.hip).
 #pragma once
 
 #include <type_traits>

@@ -31,7 +31,8 @@
 // Infinities: x = inf splits into (inf, 0, 0), whose small partial products would be inf * 0 = NaN. A
 // workgroup that has met one (or a number that rounds to one in bf16) sweeps its tiles again, with
 // every infinite h taken as 0 in the small products: h h alone then gives what the fp32 product
-// gives. (A branch in each tile instead cost the backward kernels up to 200 spilled registers.)
+// gives; where waves have no barrier in a sweep (pa_mfma_f32_block.hip) each decides for itself. (A branch
+// in each tile instead cost the backward kernels up to 200 spilled registers.)
 // Masks, key bias classes, value multiplier, softclamp, causal limits and
 // the module epilogue follow the pass semantics of polyattn.h; rows left fully masked get lse = NaN
 // for k_fwd_fixup, as in the 16-bit kernels.
@@ -443,7 +444,10 @@ void launch_mfma_bwd_f32(const GradDev& G, hipStream_t s) {
     const PassDev& P = G.f;
     // (unit counts in 64 bits: a product past 2^31 must not wrap into the small-grid test)
     const int64_t qunits = (int64_t)P.batch * P.heads, kunits = (int64_t)P.batch * G.hk;
-    {
+    const int64_t qblocks = qunits * ((P.nq + 31) / 32);
+    if (mfma_f32_block_applies(P, qblocks)) {
+        launch_mfma_bwd_f32_dq_block(G, qblocks, s);
+    } else {
         const int r = f32_rows(qunits, P.nq, P.dim, P.causal != 0);
         ProfScope ps(f32_split(r, P.dim) ? "mfma_bwd_f32_dq_split" : "mfma_bwd_f32_dq", s);
         PA_F32_LAUNCH(k_mfma_bwd_f32_dq, r, P.nq, qunits, G);
@@ -464,7 +468,11 @@ bool mfma_fwd_f32_supported(const PassDev& P) {
 }
 
 void launch_mfma_fwd_f32(const PassDev& P, hipStream_t s) {
-    const int64_t units = (int64_t)P.batch * P.heads;
+    const int64_t units = (int64_t)P.batch * P.heads, blocks = units * ((P.nq + 31) / 32);
+    if (mfma_f32_block_applies(P, blocks)) {
+        launch_mfma_fwd_f32_block(P, blocks, s);
+        return;
+    }
     const int r = f32_rows(units, P.nq, P.dim, P.causal != 0);
     ProfScope ps(f32_split(r, P.dim) ? "mfma_fwd_f32_split" : "mfma_fwd_f32", s);
     PA_F32_LAUNCH(k_mfma_fwd_f32, r, P.nq, units, P);

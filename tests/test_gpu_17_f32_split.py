@@ -152,3 +152,40 @@ def test_accuracy_of_extreme_magnitudes(scale):
     got = [out.detach(), *torch.autograd.grad(out, ts, do.to(dev()))]
     for a, b in zip(got, _pass64(q, k, v, do)):
         assert ((a.double().cpu() - b).norm() / b.norm()).item() < 2e-6
+
+
+@param("n", (225, 256, 257, 300))
+@param("causal", (False, True))
+@param("vmul", (False, True))
+def test_one_block_per_workgroup(n, causal, vmul):
+    """Head dim 128 in small grids of eight tiles or more (forward and dQ: four waves of a workgroup on
+    one row block): one row past a tile, waves with two and with three tiles, and causal blocks
+    that leave waves without any; GQA, key bias."""
+    q = randn((1, 4, n, 128), torch.float32, 30)
+    k, v, m = (randn((1, 2, n, 128), torch.float32, s) for s in (31, 32, 33))
+    bias = randn((1, 2, n), torch.float32, 34)
+    check(run_pass(q, k, v, vmul=m if vmul else None, bias=bias, causal=causal), torch.float32,
+          f"one block n={n} causal={causal} vmul={vmul}")
+
+
+@param("causal", (False, True))
+def test_one_block_masks_and_softclamp(causal):
+    n = 270
+    q, k, v = (randn((2, 2, n, 128), torch.float32, s) for s in (35, 36, 37))
+    km = torch.ones(2, n, dtype=torch.bool)
+    km[0, :70] = False
+    km[1, 200:] = False
+    check(run_pass(q, k, v, key_mask=km, causal=causal), torch.float32, f"one block masked causal={causal}")
+    check(run_pass(q, k, v, causal=causal, softclamp=2.0), torch.float32, f"one block softclamp causal={causal}")
+
+
+def test_one_block_accuracy():
+    """test_accuracy_against_64_bits at head dim 128 and as many blocks as CUs."""
+    from poly_attention import _ops
+
+    q, k, v, do = (randn((1, 8, 1024, 128), torch.float32, s) for s in (38, 39, 40, 41))
+    ts = [t.to(dev()).requires_grad_() for t in (q, k, v)]
+    out, _ = _ops.attn_pass(*ts, causal=True)
+    got = [out.detach(), *torch.autograd.grad(out, ts, do.to(dev()))]
+    for a, b in zip(got, _pass64(q, k, v, do)):
+        assert ((a.double().cpu() - b).norm() / b.norm()).item() < 2e-6
