@@ -377,10 +377,9 @@ constexpr int kKvStages = 3;
 // XV: the values are v * vmul (GradDev::xv, xm) and dv and dvmul are formed from their gradient.  A
 // template argument: as a run-time test the epilogue's registers cost every pass 3% of this kernel.
 //
-// NG = 2 (small grids at head dim 64): two groups of four waves share the workgroup's keys, group g
+// NG = 2 (head dim 64, two_wave_groups): two groups of four waves share the workgroup's keys, group g
 // taking the query tiles g, g + 2, ... with two LDS stages each; the groups' dK, dV and dbias are
-// added at the end.  (Head dim 128 holds 350 registers a
-// lane: one wave per SIMD.)
+// added at the end.  (Head dim 128 holds 350 registers a lane: one wave per SIMD.)
 template <typename T, int D, int NG, bool CAUSAL, bool SOFTCLAMP, bool HAS_BIAS, bool XV>
 __global__ __launch_bounds__(kBwdThreads * NG, D == 64 ? 2 : 1) void k_mfma_bwd_dkv_dma(GradDev G) {
     using M = Mma<T>;
@@ -1034,14 +1033,14 @@ __global__ __launch_bounds__(kBwdThreads, D == 64 ? 2 : 1) void k_mfma_bwd_dq(Gr
 // converts the tile's key bias into accumulator seeds (bias / scale; log2 domain with
 // softclamp), so that P^T = exp2(scale*log2e*S^T - lse*log2e).  Three workgroups per CU at
 // head dim 64 (the register budget fits without spills).
-// NG groups of four waves share the workgroup's queries, as in k_mfma_fwd_dma: with NG = 2 (head dim
-// 128, and small grids at 64) group g takes the key tiles g, g + 2, ..., two LDS stages each, and
-// the groups' dQ are added at the end.  Head dim 128, causal: 97 -> 79 us
-// at 2 x 16 heads x 2048, 632 -> 489 at 4 x 16 x 4096.
+// NG groups of four waves share the workgroup's queries, as in k_mfma_fwd_dma: with NG = 2
+// (two_wave_groups) group g takes the key tiles g, g + 2, ..., two LDS stages each, and the groups' dQ
+// are added at the end.  Head dim 128, causal: 97 -> 79 us at 2 x 16 heads x 2048, 632 -> 489 at
+// 4 x 16 x 4096.
 // (two workgroups per CU with softclamp: at three, 27 to 62 of its registers spill)
 template <typename T, int D, int NG, bool CAUSAL, bool SOFTCLAMP, bool HAS_BIAS>
-__global__ __launch_bounds__(kBwdThreads * NG, NG == 1 && !SOFTCLAMP ? 3 : 2) void k_mfma_bwd_dq_dma(GradDev G) {
-    static_assert(D == 64 || NG == 2, "one group of head dim 128 leaves a SIMD a single wave");
+__global__ __launch_bounds__(kBwdThreads * NG, NG == 2 ? 2 : D == 128 ? 1 : SOFTCLAMP ? 2 : 3)
+void k_mfma_bwd_dq_dma(GradDev G) {
     constexpr int NSTG = NG == 1 ? kKvStages : 4;
     using M = Mma<T>;
     typedef typename M::frag frag;
@@ -1508,15 +1507,6 @@ static bool bwd_dq_dma_ok(const GradDev& G) {
     return true;
 }
 
-// Head dim 64: workgroups of two groups of waves where those of one leave the chip idle, or, in causal
-// grids, where the last workgroups run long alone.  dQ / dK/dV us, one group -> two, by 128-row
-// workgroups: causal 128 (1 x 4 heads x 4096) 76 / 85 -> 58 / 71, 256 (4 x 8 x 1000) 28 / 31 ->
-// 25 / 28, 512 (2 x 8 x 4096) 85 / 100 -> 73 / 89, 1024 (4 x 16 x 2048) 79 / 89 -> 84 / 104;
-// not causal 64 (1 x 8 x 1024) 27 / 27 -> 23 / 25, 384 (16 x 8 x 300) 21 / 20 -> 27 / 29.
-static bool bwd_two_groups(uint32_t workgroups, bool causal) {
-    return workgroups <= (causal ? 512u : 128u);
-}
-
 template <typename T, int D, bool C, bool S, bool V, bool B>
 static void launch_dq(const GradDev& G, hipStream_t s) {
     const PassDev& P = G.f;
@@ -1526,13 +1516,10 @@ static void launch_dq(const GradDev& G, hipStream_t s) {
     // fit in LDS)
     if constexpr (D != 256) {
         if (!V && PA_BWD_DMA && bwd_dq_dma_ok(G)) {
-            if constexpr (D == 64) {
-                if (!bwd_two_groups(grid.x, C)) {
-                    hipLaunchKernelGGL((k_mfma_bwd_dq_dma<T, D, 1, C, S, B>), grid, dim3(kBwdThreads), 0, s, G);
-                    return;
-                }
-            }
-            hipLaunchKernelGGL((k_mfma_bwd_dq_dma<T, D, 2, C, S, B>), grid, dim3(2 * kBwdThreads), 0, s, G);
+            if (two_wave_groups(false, D, C, (int64_t)P.batch * P.heads, P.nq, P.nk))
+                hipLaunchKernelGGL((k_mfma_bwd_dq_dma<T, D, 2, C, S, B>), grid, dim3(2 * kBwdThreads), 0, s, G);
+            else
+                hipLaunchKernelGGL((k_mfma_bwd_dq_dma<T, D, 1, C, S, B>), grid, dim3(kBwdThreads), 0, s, G);
             return;
         }
     }
@@ -1568,7 +1555,9 @@ static void launch_bwd_t(const GradDev& G0, hipStream_t s) {
         bool done = false;
         if constexpr (D != 256) {  // head dim 256: the register-staged kernel only
             if (kv_dma) {
-                launch_dkv_dma<T, D, C, S, B>(G, grid, D == 64 && bwd_two_groups(grid.x, C), s);
+                const bool two = D == 64 && two_wave_groups(false, D, C, (int64_t)P.batch * G.hk, P.nk,
+                                                            (int64_t)P.nq * (P.heads / G.hk));
+                launch_dkv_dma<T, D, C, S, B>(G, grid, two, s);
                 done = true;
             }
         }

@@ -590,9 +590,9 @@ struct DmaTile {
 // stages are 128 KB, and in grids of fewer workgroups than the chip holds; and it halves the
 // longest serial chain of a causal grid, its last queries' tiles.  Measured, us per level, one
 // group -> two: d = 128, causal, 2 x 16 heads x 2048 68 -> 56, 4 x 16 x 4096 434 -> 340; d = 64,
-// causal, 2 x 8 x 4096 86 -> 57.
+// causal, 2 x 8 x 4096 86 -> 57.  Where the line lies, with both sides: two_wave_groups (pa_order.h).
 template <typename T, int D, int KB, int QB, int NG, bool CAUSAL, bool SOFTCLAMP, bool HAS_BIAS>
-__global__ __launch_bounds__(kFwdThreads * NG, 2) void k_mfma_fwd_dma(PassDev P) {
+__global__ __launch_bounds__(kFwdThreads * NG, D == 128 && NG == 1 ? 1 : 2) void k_mfma_fwd_dma(PassDev P) {
     using TL = DmaTile<D, KB>;
     constexpr int BN = TL::BN, NL = TL::NL, BM = kFwdBM * QB;
     // the key bias enters the scores as bias / scale (so that scale*log2e*(s + bias/scale) is the
@@ -1457,21 +1457,15 @@ static void launch_t(const PassDev& P, hipStream_t s) {
         if (!V && dma_ok(P, 32 * KB)) {
             const int64_t units = (int64_t)P.heads * P.batch;
             auto wgs = [&](int rows) { return (uint32_t)(units * ((P.nq + rows - 1) / rows)); };
-            if constexpr (D == 64) {
-                // 256-query workgroups of one group where they fill the chip (two a CU), else
-                // 128-query workgroups of two.  us at 64 / 256 / 512 256-query workgroups, causal
-                // (1 x 4, 2 x 8, 8 x 16 heads x N = 4096, 4096, 1024): 82 / 86 / 35 one group,
-                // 46 / 57 / 45 two; not causal at 32 / 256 (8, 64 heads x 1000): 27 / 33, 18 / 36
-                const uint32_t w2 = wgs(2 * kFwdBM);
-                if (w2 >= (C ? 384u : 192u))
-                    hipLaunchKernelGGL((k_mfma_fwd_dma<T, D, KB, 2, 1, C, S, B>), dim3(w2), dim3(kFwdThreads), 0, s, P);
-                else
-                    hipLaunchKernelGGL((k_mfma_fwd_dma<T, D, KB, 1, 2, C, S, B>), dim3(wgs(kFwdBM)),
-                                       dim3(2 * kFwdThreads), 0, s, P);
-            } else {
+            // 128-query workgroups of two groups of waves, or of one: with 256 queries at head dim
+            // 64 (two query blocks a wave), with 128 at 128
+            constexpr int QB = D == 64 ? 2 : 1;
+            if (two_wave_groups(true, D, C, units, P.nq, P.nk))
                 hipLaunchKernelGGL((k_mfma_fwd_dma<T, D, KB, 1, 2, C, S, B>), dim3(wgs(kFwdBM)),
                                    dim3(2 * kFwdThreads), 0, s, P);
-            }
+            else
+                hipLaunchKernelGGL((k_mfma_fwd_dma<T, D, KB, QB, 1, C, S, B>), dim3(wgs(QB * kFwdBM)),
+                                   dim3(kFwdThreads), 0, s, P);
             return;
         }
     }
