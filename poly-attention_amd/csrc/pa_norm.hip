@@ -5,6 +5,7 @@
 // row back; the backward writes dx and accumulates the weight gradient per workgroup into a
 // fixed partial row, summed afterwards in a fixed order (deterministic, no atomics).
 #include <algorithm>
+#include <type_traits>
 
 #include "pa_common.h"
 #include "pa_launch.h"
@@ -120,47 +121,76 @@ __device__ __forceinline__ void fill_trig(const RmsDev& R, float2* tab, uint32_t
     __syncthreads();
 }
 
-// cos / sin of the E features d0.. of row r (of the run starting at `first`, in slot row u), as
-// used by the rotation: from the table or evaluated here
-template <int E>
-__device__ __forceinline__ void row_trig(const RmsDev& R, const float2* tab, int u, uint32_t first,
-                                         uint32_t r, uint32_t pos, int d0, float2 (&t)[E]) {
-    if (R.trig) {
+// where a kernel's rotation takes its cos / sin from: a template argument, since the code of both ways
+// and the table's LDS cost the norms without a table (fewer than 4 heads, contiguous heads) up to
+// 45%: 4 x 16 heads x 4096, d = 64, bf16, contiguous, forward 42 us before the table, 61 with both
+// ways in one kernel, 44 like this; 2 heads x 512 12.2, 15.0 and 13.0.
+enum { kRopeNone, kRopeRows, kRopeTable, kRopeEither };  // either: by R.trig
+
+template <int ROPE>
+__device__ __forceinline__ bool rope_table(const RmsDev& R) {
+    return ROPE == kRopeTable || (ROPE == kRopeEither && R.trig);
+}
+
+// f(get), get(e) the cos / sin of feature d0 + e of row r (of the run starting at `first`, in slot row
+// u): all read from the table, or evaluated, at once; with PAIRS evaluated as they are used (the
+// forward's array of eight took it from 119 to 135 registers; the 16-bit backward, three waves a
+// SIMD either way, is 5% faster with it)
+template <int ROPE, int E, bool PAIRS, class F>
+__device__ __forceinline__ void with_trig(const RmsDev& R, const float2* tab, int u, uint32_t first,
+                                          uint32_t r, uint32_t pos, int d0, F f) {
+    float2 t[E];
+    if (rope_table<ROPE>(R)) {
         const int k = (int)(R.fd_h.div(r) - R.fd_h.div(first));
         const float2* p = tab + (u * R.trig + k) * R.rot_dim + d0;
 #pragma unroll
         for (int e = 0; e < E; ++e)
             if (d0 + e < R.rot_dim) t[e] = p[e];
+    } else if (PAIRS) {
+        f([&](int e) __attribute__((always_inline)) { return rope_trig(R, pos, d0 + e); });
+        return;
     } else {
 #pragma unroll
         for (int e = 0; e < E; ++e)
             if (d0 + e < R.rot_dim) t[e] = rope_trig(R, pos, d0 + e);
     }
+    f([&](int e) __attribute__((always_inline)) { return t[e]; });
+}
+
+// a result in fp32 of its own.  Every kernel of the norms gives the same bits: sums of products are
+// written as the fused operations that they are, and an fp16 conversion is not fused into one (a
+// compiler does that where no branch lies between).
+template <typename T>
+__device__ __forceinline__ float own(float x) {
+    if (std::is_same<T, f16>::value) asm("" : "+v"(x));
+    return x;
 }
 
 // rotary embedding of the E features d0.. of one row in place (fp32 math on the rounded
 // norm output t, one rounding when stored): y[2i] = t[2i] cos a[2i] - t[2i+1] sin a[2i],
 // y[2i+1] = t[2i+1] cos a[2i+1] + t[2i] sin a[2i+1]
-template <int E>
-__device__ __forceinline__ void rope_fwd(const RmsDev& R, int d0, const float2 (&c)[E], float (&t)[E]) {
+template <typename T, int E, class Get>
+__device__ __forceinline__ void rope_fwd(const RmsDev& R, int d0, Get get, float (&t)[E]) {
 #pragma unroll
     for (int e = 0; e < E; e += 2) {
         if (d0 + e >= R.rot_dim) break;
+        const float2 a = get(e), b = get(e + 1);
         const float t0 = t[e], t1 = t[e + 1];
-        t[e] = t0 * c[e].x - t1 * c[e].y;
-        t[e + 1] = t1 * c[e + 1].x + t0 * c[e + 1].y;
+        t[e] = own<T>(fmaf(t0, a.x, -(t1 * a.y)));
+        t[e + 1] = own<T>(fmaf(t1, b.x, t0 * b.y));
     }
 }
 
 // the gradient of t from the gradient g of the rotated row (the transposed rotation)
-template <int E>
-__device__ __forceinline__ void rope_bwd(const RmsDev& R, int d0, const float2 (&c)[E], float (&g)[E]) {
+template <typename T, int E, class Get>
+__device__ __forceinline__ void rope_bwd(const RmsDev& R, int d0, Get get, float (&g)[E]) {
 #pragma unroll
     for (int e = 0; e < E; e += 2) {
         if (d0 + e >= R.rot_dim) break;
+        const float2 a = get(e), b = get(e + 1);
         const float g0 = g[e], g1 = g[e + 1];
-        g[e] = g0 * c[e].x + g1 * c[e + 1].y;
-        g[e + 1] = g1 * c[e + 1].x - g0 * c[e].y;
+        g[e] = own<T>(fmaf(g0, a.x, g1 * b.y));
+        g[e + 1] = own<T>(fmaf(g1, b.x, -(g0 * a.y)));
     }
 }
 
@@ -186,7 +216,7 @@ __device__ __forceinline__ uint32_t rstd_index(const RmsDev& R, uint32_t b, uint
 
 // y = round(x * rsqrt(mean(x^2) + eps) * w); rstd saved per row.  Each row group handles
 // kRmsU rows per pass, their loads issued together (memory-level parallelism).
-template <typename T, int LPR, bool ROPE>
+template <typename T, int LPR, int ROPE>
 __device__ __forceinline__ void rms_fwd_rows(const RmsDev& R) {
     constexpr int E = RVec<T>::n;
     constexpr int RPB = kRmsThreads / LPR;  // row groups per block
@@ -197,10 +227,10 @@ __device__ __forceinline__ void rms_fwd_rows(const RmsDev& R) {
 #pragma unroll
     for (int e = 0; e < E; ++e) w[e] = (R.w && dok) ? load_any(R.w, R.wdt, d0 + e) : 1.f;
     const uint32_t step = gridDim.x * RPB;
-    __shared__ float2 tab[ROPE ? kTrigMax : 1];
+    __shared__ float2 tab[ROPE >= kRopeTable ? kTrigMax : 1];
     for (uint32_t first = blockIdx.x * RPB; first < R.rows; first += step * kRmsU) {
         const uint32_t r0 = first + rg;
-        if (ROPE && R.trig) fill_trig(R, tab, first, step);
+        if (rope_table<ROPE>(R)) fill_trig(R, tab, first, step);
         float x[kRmsU][E];
         uint32_t b[kRmsU], h[kRmsU], i[kRmsU];
 #pragma unroll
@@ -226,9 +256,8 @@ __device__ __forceinline__ void rms_fwd_rows(const RmsDev& R) {
                     // the norm output is a tensor of T before the rotation
 #pragma unroll
                     for (int e = 0; e < E; ++e) y[e] = round_to<T>(y[e]);
-                    float2 c[E];
-                    row_trig<E>(R, tab, u, first + u * step, r, i[u], d0, c);
-                    rope_fwd<E>(R, d0, c, y);
+                    with_trig<ROPE, E, true>(R, tab, u, first + u * step, r, i[u], d0,
+                                             [&](auto get) __attribute__((always_inline)) { rope_fwd<T, E>(R, d0, get, y); });
                 }
                 store_row<T>(R.y.at<T>(b[u], h[u], i[u]) + d0, y);
             }
@@ -237,8 +266,9 @@ __device__ __forceinline__ void rms_fwd_rows(const RmsDev& R) {
     }
 }
 
-template <typename T, int LPR, bool ROPE>
-__global__ __launch_bounds__(kRmsThreads) void k_rms_fwd(RmsDev R) {
+// (four waves per SIMD: 129 registers without the bound at LPR = 16 with rotary)
+template <typename T, int LPR, int ROPE>
+__global__ __launch_bounds__(kRmsThreads, 4) void k_rms_fwd(RmsDev R) {
     rms_fwd_rows<T, LPR, ROPE>(R);
 }
 
@@ -250,14 +280,14 @@ struct RmsMany {
     RmsDev it[PA_RMS_MAX_ITEMS];
 };
 
-template <typename T, int LPR, bool ROPE>
-__global__ __launch_bounds__(kRmsThreads) void k_rms_fwd_many(RmsMany M) {
+template <typename T, int LPR, int ROPE>
+__global__ __launch_bounds__(kRmsThreads, 4) void k_rms_fwd_many(RmsMany M) {
     rms_fwd_rows<T, LPR, ROPE>(M.it[blockIdx.y]);
 }
 
 // dx = rstd * (g - xhat * mean(g * xhat)), g = dy * w, xhat = x * rstd; the block's weight
 // gradient partial sum_rows dy * xhat goes to partial[blockIdx.x]
-template <typename T, int LPR, bool ROPE>
+template <typename T, int LPR, int ROPE>
 __device__ __forceinline__ void rms_bwd_rows(const RmsDev& R) {
     constexpr int E = RVec<T>::n;
     constexpr int RPB = kRmsThreads / LPR;
@@ -273,10 +303,10 @@ __device__ __forceinline__ void rms_bwd_rows(const RmsDev& R) {
         acc[e] = 0.f;
     }
     const uint32_t step = gridDim.x * RPB;
-    __shared__ float2 tab[ROPE ? kTrigMax : 1];
+    __shared__ float2 tab[ROPE >= kRopeTable ? kTrigMax : 1];
     for (uint32_t first = blockIdx.x * RPB; first < R.rows; first += step * kRmsU) {
         const uint32_t r0 = first + rg;
-        if (ROPE && R.trig) fill_trig(R, tab, first, step);
+        if (rope_table<ROPE>(R)) fill_trig(R, tab, first, step);
         float x[kRmsU][E], dy[kRmsU][E], rs[kRmsU];
         uint32_t b[kRmsU], h[kRmsU], i[kRmsU];
 #pragma unroll
@@ -292,10 +322,10 @@ __device__ __forceinline__ void rms_bwd_rows(const RmsDev& R) {
             // back through the rotation: the gradient of the norm output, a tensor of T
 #pragma unroll
             for (int u = 0; u < kRmsU; ++u) {
-                float2 c[E];
                 const uint32_t r = r0 + u * step;
-                row_trig<E>(R, tab, u, first + u * step, r < R.rows ? r : first + u * step, i[u], d0, c);
-                rope_bwd<E>(R, d0, c, dy[u]);
+                with_trig<ROPE, E, E == 4>(
+                    R, tab, u, first + u * step, r < R.rows ? r : first + u * step, i[u], d0,
+                    [&](auto get) __attribute__((always_inline)) { rope_bwd<T, E>(R, d0, get, dy[u]); });
 #pragma unroll
                 for (int e = 0; e < E; ++e) dy[u][e] = round_to<T>(dy[u][e]);
             }
@@ -306,14 +336,14 @@ __device__ __forceinline__ void rms_bwd_rows(const RmsDev& R) {
 #pragma unroll
             for (int e = 0; e < E; ++e) {
                 const float xh = x[u][e] * rs[u];
-                c += dy[u][e] * w[e] * xh;
-                acc[e] += dy[u][e] * xh;
+                c = fmaf(dy[u][e] * w[e], xh, c);
+                acc[e] = fmaf(dy[u][e], xh, acc[e]);
             }
             c = row_sum<LPR>(c) * R.inv_dim;
             if (r0 + u * step < R.rows && dok) {
                 float dx[E];
 #pragma unroll
-                for (int e = 0; e < E; ++e) dx[e] = rs[u] * (dy[u][e] * w[e] - x[u][e] * rs[u] * c);
+                for (int e = 0; e < E; ++e) dx[e] = own<T>(rs[u] * fmaf(dy[u][e], w[e], -(x[u][e] * rs[u] * c)));
                 store_row<T>(R.dx.at<T>(b[u], h[u], i[u]) + d0, dx);
             }
         }
@@ -335,12 +365,12 @@ __device__ __forceinline__ void rms_bwd_rows(const RmsDev& R) {
     }
 }
 
-template <typename T, int LPR, bool ROPE>
+template <typename T, int LPR, int ROPE>
 __global__ __launch_bounds__(kRmsThreads) void k_rms_bwd(RmsDev R) {
     rms_bwd_rows<T, LPR, ROPE>(R);
 }
 
-template <typename T, int LPR, bool ROPE>
+template <typename T, int LPR, int ROPE>
 __global__ __launch_bounds__(kRmsThreads) void k_rms_bwd_many(RmsMany M) {
     rms_bwd_rows<T, LPR, ROPE>(M.it[blockIdx.y]);
 }
@@ -443,7 +473,7 @@ static int rms_setup(const pa_rmsnorm* p, RmsDev& R, bool bwd) {
     return PA_OK;
 }
 
-template <typename T, bool ROPE>
+template <typename T, int ROPE>
 static void rms_launch_r(const RmsDev& R, bool bwd, hipStream_t s) {
     const dim3 grid(rms_blocks(R));
 #define PA_RMS_CASE(L)                                                                          \
@@ -465,8 +495,9 @@ static void rms_launch_r(const RmsDev& R, bool bwd, hipStream_t s) {
 
 template <typename T>
 static void rms_launch(const RmsDev& R, bool bwd, hipStream_t s) {
-    if (R.ang) rms_launch_r<T, true>(R, bwd, s);
-    else rms_launch_r<T, false>(R, bwd, s);
+    if (!R.ang) rms_launch_r<T, kRopeNone>(R, bwd, s);
+    else if (R.trig) rms_launch_r<T, kRopeTable>(R, bwd, s);
+    else rms_launch_r<T, kRopeRows>(R, bwd, s);
 }
 
 int launch_rms_fwd(const pa_rmsnorm* p, hipStream_t s) {
@@ -495,7 +526,7 @@ static int rms_many_setup(const pa_rmsnorm* items, int count, bool bwd, RmsMany&
     return blocks;
 }
 
-template <typename T, bool ROPE>
+template <typename T, int ROPE>
 static void rms_many_launch_r(const RmsMany& M, dim3 grid, bool bwd, hipStream_t s) {
 #define PA_RMS_CASE(L)                                                                               \
     case L:                                                                                          \
@@ -514,13 +545,20 @@ static void rms_many_launch_r(const RmsMany& M, dim3 grid, bool bwd, hipStream_t
 #undef PA_RMS_CASE
 }
 
-static void rms_many_launch(const RmsMany& M, int dtype, dim3 grid, bool bwd, hipStream_t s) {
-    const bool rope = M.it[0].ang != nullptr;
-#define PA_RMS_T(T) (rope ? rms_many_launch_r<T, true>(M, grid, bwd, s) : rms_many_launch_r<T, false>(M, grid, bwd, s))
-    if (dtype == PA_F32) PA_RMS_T(float);
-    else if (dtype == PA_F16) PA_RMS_T(f16);
-    else PA_RMS_T(bf16);
-#undef PA_RMS_T
+template <typename T>
+static void rms_many_launch_t(const RmsMany& M, int count, dim3 grid, bool bwd, hipStream_t s) {
+    int tables = 0;
+    for (int k = 0; k < count; ++k) tables += M.it[k].trig != 0;
+    if (!M.it[0].ang) rms_many_launch_r<T, kRopeNone>(M, grid, bwd, s);
+    else if (tables == count) rms_many_launch_r<T, kRopeTable>(M, grid, bwd, s);
+    else if (tables == 0) rms_many_launch_r<T, kRopeRows>(M, grid, bwd, s);
+    else rms_many_launch_r<T, kRopeEither>(M, grid, bwd, s);
+}
+
+static void rms_many_launch(const RmsMany& M, int dtype, int count, dim3 grid, bool bwd, hipStream_t s) {
+    if (dtype == PA_F32) rms_many_launch_t<float>(M, count, grid, bwd, s);
+    else if (dtype == PA_F16) rms_many_launch_t<f16>(M, count, grid, bwd, s);
+    else rms_many_launch_t<bf16>(M, count, grid, bwd, s);
 }
 
 int launch_rms_fwd_many(const pa_rmsnorm* items, int count, hipStream_t s) {
@@ -530,7 +568,7 @@ int launch_rms_fwd_many(const pa_rmsnorm* items, int count, hipStream_t s) {
     const int blocks = rms_many_setup(items, count, false, M);
     if (blocks < 0) return blocks;
     ProfScope ps("rms_fwd_many", s);
-    rms_many_launch(M, items[0].x.dtype, dim3(blocks, count), false, s);
+    rms_many_launch(M, items[0].x.dtype, count, dim3(blocks, count), false, s);
     return PA_OK;
 }
 
@@ -558,7 +596,7 @@ int launch_rms_many(const pa_rmsnorm* items, int count, bool bwd, hipStream_t s)
     }
     {
         ProfScope ps(bwd ? "rms_bwd" : "rms_fwd", s);
-        rms_many_launch(M, items[0].x.dtype, grid, bwd, s);
+        rms_many_launch(M, items[0].x.dtype, count, grid, bwd, s);
     }
     if (dw) {
         ProfScope ps("rms_dw", s);

@@ -126,3 +126,26 @@ def test_prefill_rotates_keys_as_the_module(order, dtype, freqs_too, monkeypatch
             else:
                 err = (got.float() - want.float()).abs()
                 assert (err <= torch.finfo(dtype).eps * want.float().abs() + 1e-6).all()
+
+
+@param("dtype", (torch.bfloat16, torch.float32))
+@param("heads", ((4, 8), (2, 3), (8, 2)))
+def test_layer_norms_with_and_without_a_table(dtype, heads):
+    """The norms of a layer in one launch where every tensor has the cos / sin table (4 heads and more),
+    none has, and one has (kv heads): the same bits as one by one, forward and backward."""
+    from poly_attention import _ops
+
+    n, d = 37, 64
+    ang = torch.arange(n, device=dev()).float()[:, None] * randn((d,), torch.float32, 1).to(dev()).abs()
+    xs = [randn((2, n, h, d), dtype, 2 + h).to(dev()).transpose(1, 2) for h in heads]
+    ws = [(1 + 0.1 * randn((d,), torch.float32, 20 + h)).to(dtype).to(dev()) for h in heads]
+    dys = [randn((2, n, h, d), dtype, 40 + h).to(dev()).transpose(1, 2) for h in heads]
+    got = []
+    for layer in (True, False):
+        ins = [t.detach().requires_grad_() for t in (*xs, *ws)]
+        x, w = ins[:2], ins[2:]
+        ys = (_ops.rms_norm_layer(x, w, [1e-6] * 2, ang) if layer else
+              [_ops.rms_norm(a, b, 1e-6, ang) for a, b in zip(x, w)])
+        got.append([*ys, *torch.autograd.grad(ys, x, dys)])
+    for a, b in zip(*got):
+        assert torch.equal(a, b)
