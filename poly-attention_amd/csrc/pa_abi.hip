@@ -206,7 +206,12 @@ size_t fwd_key_bytes(const pa_pass& f) {
            align256(kheads * 2 * sizeof(int32_t));
 }
 
-size_t fwd_ws_bytes(const pa_pass& f) { return fwd_key_bytes(f) + value_bytes(f); }
+// ... and the effective value, where the rows are long enough to pay for forming it (us with the
+// register-staged kernel, which multiplies on the way, and with the fold: 16 heads x 128, d = 64
+// 9.8 / 10.6, x 200 12.2 / 11.3; d = 128, 64 heads x 64 10.5 / 11.1, x 100 13.6 / 12.6)
+size_t fwd_value_bytes(const pa_pass& f) { return f.nk > (f.dim == 64 ? 128 : 64) ? value_bytes(f) : 0; }
+
+size_t fwd_ws_bytes(const pa_pass& f) { return fwd_key_bytes(f) + fwd_value_bytes(f); }
 
 // [D | lse | 1/c1] per query row; with an epilogue the gradient reaching the pass output;
 // masked passes add the key term (with a key mask), the per-head fully-masked-row sums, the
@@ -404,7 +409,7 @@ int pa_attn_pass_fwd(const pa_pass* p, void* stream) {
                 Pm.km.p = nullptr;
                 Pm.live = live;
             }
-            if (value_bytes(*p)) {
+            if (fwd_value_bytes(*p)) {
                 PassDev Pv = Pm;
                 Pv.v = value_view(*p, w + fwd_key_bytes(*p));
                 Pv.vmul.p = nullptr;
