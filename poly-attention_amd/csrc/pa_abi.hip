@@ -207,8 +207,8 @@ size_t fwd_key_bytes(const pa_pass& f) {
 }
 
 // ... and the effective value, where the rows are long enough to pay for forming it (us with the
-// register-staged kernel, which multiplies on the way, and with the fold: 16 heads x 128, d = 64
-// 9.8 / 10.6, x 200 12.2 / 11.3; d = 128, 64 heads x 64 10.5 / 11.1, x 100 13.6 / 12.6)
+// register-staged kernel, which multiplies on the way, and with the fold, 16 heads: d = 64, x 128
+// 9.8 / 10.6, x 200 13.2 / 12.0; d = 128, x 64 10.3 / 10.9, x 128 14.2 / 12.4)
 size_t fwd_value_bytes(const pa_pass& f) { return f.nk > (f.dim == 64 ? 128 : 64) ? value_bytes(f) : 0; }
 
 size_t fwd_ws_bytes(const pa_pass& f) { return fwd_key_bytes(f) + fwd_value_bytes(f); }

@@ -223,10 +223,12 @@ __global__ __launch_bounds__(kBwdThreads, D == 64 ? 2 : 1) void k_mfma_bwd_dkv(G
             kv_store<T, D>(st, sQ, sO, sQt, sOt, sL, sD);
             __syncthreads();
             if (PREFETCH && t + 1 < ntiles) kv_load<T, D>(qs, q0 + kKvBQ, st);
-            // head dim 256, not causal: the two query halves one after the other (unrolled, the
-            // scheduler kept both halves' temporaries live: 479 against 106 spilled registers,
-            // 3.75 against 1.80 ms per launch at N = 2048); causal, unrolled was faster
-#pragma unroll(D == 256 && !CAUSAL ? 1 : 2)
+            // head dim 256, not causal or with softclamp: the two query halves one after the other
+            // (unrolled, the scheduler kept both halves' temporaries live: 479 against 106 spilled
+            // registers, 3.75 against 1.80 ms per launch at N = 2048; causal with softclamp and a
+            // bias 554 against 79, a pass's backward at 8 heads x 1000 490 against 292 us); causal
+            // without softclamp, unrolled was faster
+#pragma unroll(D == 256 && (!CAUSAL || SOFTCLAMP) ? 1 : 2)
             for (int qb = 0; qb < 2; ++qb) {
                 const int qbase = q0 + qb * 32;
                 if (CAUSAL && qbase + 31 < kw0) continue;  // every query precedes every key
