@@ -154,8 +154,9 @@ typedef struct pa_pass {
     const pa_epilogue* epi;  /* optional module epilogue (NULL: none) */
     /* Optional forward workspace of pa_attn_pass_fwd_workspace() bytes (ignored by the
      * backward): with it a key-masked pass folds its key mask into a per-key term, a pass with
-     * a value multiplier the product v * vmul into one tensor, and takes the faster forward
-     * kernel; without it the results are the same. */
+     * a value multiplier and rows long enough to gain by it the product v * vmul into one
+     * tensor, and takes the faster forward kernel; without it the results are the same up to
+     * the order of summation. */
     void*   workspace;
     size_t  workspace_bytes;
     const pa_qk_norm* norm;  /* optional q / k norms on load (NULL: none; forward only) */
